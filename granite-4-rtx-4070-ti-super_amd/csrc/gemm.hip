@@ -40,10 +40,7 @@
 // does not depend on the matrix cores' internal k order. The 16 x 16 f32
 // result: lane l holds rows 4 (l / 16) + i, column l % 16.
 
-#include "g4_common.h"
-#include "g4_hw.h"
-#include "g4_math.h"
-#include "granite4_layerops.h"
+#include "gemm_common.h"
 
 #include <cmath>
 #include <cstdio>
@@ -62,53 +59,6 @@ constexpr int kGStage = (kGBM + kGBN) * kGBK;  // bytes per pipeline stage
 #endif
 constexpr int kGStages = G4_GEMM_STAGES;
 constexpr int kEP = 68;  // f32 pitch of the epilogue's LDS staging rows
-
-enum : int {
-  kEpiBf16 = GRANITE4_GEMM_BF16,
-  kEpiF32 = GRANITE4_GEMM_F32,
-  kEpiResidual = GRANITE4_GEMM_RESIDUAL,
-  kEpiSwiglu = 3
-};
-
-typedef int v8i __attribute__((ext_vector_type(8)));
-typedef unsigned v4u __attribute__((ext_vector_type(4)));
-typedef float v4f __attribute__((ext_vector_type(4)));
-
-struct GemmArgs {
-  const uint8_t* A;
-  int lda;
-  const float* a_scale;  // device: the activation's per-tensor scale
-  const uint8_t* W;
-  int M, N, K;  // N: weight rows (swiglu: 2I)
-  int I;        // swiglu: act columns
-  Granite4GemmEpilogue ep;
-  float* partials;  // swiglu: [gridDim.x] max |act|
-  int mt, nt;       // tile counts along M and N
-  bool vec_out;     // 16-byte output rows (pitch and width multiples of 8)
-  bool xcd_order;   // tiles renumbered per XCD (xcd_tile0)
-  // Skinny kBf16 only (gemm_rows_split): when seg_out[0] is set, column n of
-  // segment s (ep.seg1 / ep.seg2 bounds) goes to seg_out[s][m * seg_ld[s] +
-  // n - start of s] instead of ep.out_bf16.
-  uint16_t* seg_out[3];
-  int seg_ld[3];
-};
-
-// Workgroups are handed to the 8 XCDs round-robin by id (id % 8), each XCD
-// with its own L2. The first tile of workgroup b is renumbered so that
-// consecutive tile numbers - the M tiles of one weight column, which read the
-// same W rows - run on one XCD and share its L2 instead of each XCD fetching
-// the column: b -> (b % 8) * (g / 8) + b / 8 over the first 8 * floor(g / 8)
-// workgroups (g the grid), the identity on the rest. Tile t + g keeps the
-// same XCD as tile t.
-__device__ __forceinline__ int xcd_tile0(bool on) {
-  const int b = blockIdx.x, g = gridDim.x, full = g & ~7;
-  if (!on || b >= full) return b;
-  return (b & 7) * (full >> 3) + (b >> 3);
-}
-
-__device__ __forceinline__ float epi_scale(const Granite4GemmEpilogue& ep, int n) {
-  return n < ep.seg1 ? ep.scale0 : (n < ep.seg2 ? ep.scale1 : ep.scale2);
-}
 
 // Weight row behind tile row r (0..127) of N tile tn, or -1 past the end.
 template <int EPI, int TN = kGBN>
@@ -212,21 +162,7 @@ __device__ __forceinline__ void frag_issue(uint32_t region, int r, int lane, v4u
   y = lds_read16(row + 16u * static_cast<uint32_t>((c0 + 1) ^ chunk_swz(r)));
 }
 
-__device__ __forceinline__ v8i frag_of(const v4u& x, const v4u& y) {
-  v8i f;
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    f[i] = static_cast<int>(x[i]);
-    f[i + 4] = static_cast<int>(y[i]);
-  }
-  return f;
-}
-
 __device__ __forceinline__ void wave_lds_wait() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
-
-// Two bf16 RNE conversions in one v_cvt_pk_bf16_f32 (equal to the integer
-// rounding for every non-NaN value).
-__device__ __forceinline__ uint32_t pack_bf16_rne(float lo, float hi) { return pack_bf16_hw(lo, hi); }
 
 // Waits until at most `later` stages' loads (LPS per thread each) are in
 // flight (vmcnt counts a thread's loads in issue order).
@@ -509,8 +445,6 @@ constexpr int kBwARow = 2 * kBwK;                 // A bytes per tile row per st
 constexpr int kBwWRow = kBwK;                     // W bytes per tile row per stage
 constexpr int kBwStage = kGBM * kBwARow + kGBN * kBwWRow;  // 24 KB
 
-typedef __bf16 bf16x8_g __attribute__((ext_vector_type(8)));
-
 template <int EPI>
 __device__ __forceinline__ void bw_stage_issue(const GemmArgs& a, int m0, int tn, int k0,
                                                uint8_t* st) {
@@ -686,23 +620,6 @@ bool gemm_args_ok(const uint8_t* A, int lda, const uint8_t* W, int M, int N, int
          (reinterpret_cast<uintptr_t>(W) & 15u) == 0 &&
          static_cast<long long>(M) * lda < (1LL << 40);
 }
-
-// Whether XCD-ordered tiles (xcd_tile0) cut the L2 fills of a launch of g
-// workgroups over mt M tiles. Per round each XCD runs g / 8 tiles; the A rows
-// and W rows it fetches grow with the block of tiles it covers, bm M tiles x
-// bn N tiles, as bm + bn. XCD order gives each XCD whole columns, bm = mt
-// (up to g / 8); the plain order gives it every 8th tile: one M tile (mt <= 8)
-// or mt / 8 of them, spread over g / 8 or g / mt columns. Measured: T = 512
-// gate|up 88 -> 77 us with XCD order (4 x 16 against 1 x 64), T = 8192 the
-// plain order's 8 x 8 beats XCD order's 64 x 1 by 14-17 %.
-bool gemm_xcd_order(int mt, unsigned g) {
-  if (g < 16) return false;
-  const long long per = g / 8;
-  const long long xbm = mt < per ? mt : per, xbn = (per + mt - 1) / mt;
-  const long long pbm = mt <= 8 ? 1 : mt / 8, pbn = mt <= 8 ? per : (g + mt - 1) / mt;
-  return xbm + xbn < pbm + pbn;
-}
-
 
 // ---------------------------------------------------------------------------
 // Skinny GEMM, M <= 16 rows (a batched decode step's sessions, a short
@@ -987,6 +904,7 @@ int granite4_gemm_fp8(int out, const uint8_t* A, int lda, const float* d_a_scale
     else if (deep == 3) go(gemm_fp8_kernel<E, 64, 3>, gemm_grid<E, 64, 3>(tiles, INT_MAX));
     else go(gemm_fp8_kernel<E, 64>, gemm_grid<E, 64>(tiles, INT_MAX));
   };
+  if (M > kSkinnyMaxM && launch_gemm_tile_fp8(out, a) != 0) return launch_status("granite4_gemm_fp8");
   switch (out) {
     case GRANITE4_GEMM_BF16: run(std::integral_constant<int, kEpiBf16>{}); break;
     case GRANITE4_GEMM_F32: run(std::integral_constant<int, kEpiF32>{}); break;
@@ -1043,6 +961,7 @@ int granite4_prefill_gemm(int out, const uint16_t* A, int lda, const uint8_t* W,
     else launch_skinny<false, kEpiResidual>(a, INT_MAX);
     return launch_status("granite4_prefill_gemm");
   }
+  if (launch_gemm_tile_bf16(out, a) != 0) return launch_status("granite4_prefill_gemm");
   switch (out) {
     case GRANITE4_GEMM_BF16:
       hipLaunchKernelGGL(gemm_bf16w_kernel<kEpiBf16>,
@@ -1108,7 +1027,7 @@ int granite4_gemm_fp8_swiglu(const uint8_t* A, int lda, const float* d_a_scale,
   unsigned grid;
   if (M <= kSkinnyMaxM) {
     grid = launch_skinny<true, kEpiSwiglu>(a, kMaxPartials);
-  } else {
+  } else if ((grid = launch_gemm_tile_fp8(kEpiSwiglu, a)) == 0) {
     grid = gemm_grid<kEpiSwiglu>(tiles, kMaxPartials);
     a.xcd_order = gemm_xcd_order(a.mt, grid);
     hipLaunchKernelGGL(gemm_fp8_kernel<kEpiSwiglu>, grid, 256, 0, stream(), a);

@@ -1,0 +1,43 @@
+// gemm_tile_bf16.hip - the tile GEMM (gemm_tile.h) for bf16 activations: its
+// configurations and the choice between them.
+#include "gemm_tile.h"
+
+namespace g4 {
+namespace {
+
+// Rows x weight rows of a tile, and the costs fitted to 76 shapes (N x K of
+// q|k|v 6144 x 4096, O 4096 x 4096, down 4096 x 12800, one of gate|up 12800 x
+// 4096, 17 to 8192 rows, us; the choice by them is within 8 %, in the mean 0.3 %,
+// of the best of these). Measured against the 128 x 128 kernel of gemm.hip, us:
+// q|k|v 64 rows 52.4 -> 11.3, 512 rows 53.6 -> 28.2, 1000 rows 66.9 -> 47.0, 8192
+// rows 439 -> 285; O 64 rows 55.0 -> 10.4, 512 rows 55.2 -> 22.8, 8192 rows 308 ->
+// 208 (1.32 PFLOP/s; a library product of 8192^3 on the same card reaches
+// 1.28); down 64 rows 157 -> 22.3, 512 rows 158 -> 60.5, 8192 rows 901 -> 589.
+constexpr TileConfig<false, 8, 8, 2, 1, true> k256x256{{75.48f, 24.40f, -18.93f}};
+constexpr TileConfig<false, 8, 4, 3, 1, true> k256x128{{44.77f, 12.50f, -6.99f}};
+constexpr TileConfig<false, 4, 6, 4, 1, true> k128x192{{35.10f, 10.14f, -4.51f}};
+constexpr TileConfig<false, 4, 4, 3, 2, true> k128x128{{22.34f, 11.67f, -7.56f}};
+constexpr TileConfig<false, 4, 3, 3, 2, false> k128x96{{19.94f, 7.63f, -2.81f}};
+constexpr TileConfig<false, 2, 4, 3, 2, true> k64x128{{15.63f, 7.11f, -4.25f}};
+constexpr TileConfig<false, 2, 3, 4, 2, false> k64x96{{13.89f, 4.94f, -1.22f}};
+constexpr TileConfig<false, 2, 2, 4, 2, false> k64x64{{11.36f, 3.00f, -0.73f}};
+constexpr TileConfig<false, 1, 2, 6, 2, false> k32x64{{8.40f, 2.10f, 0.47f}};
+constexpr TileConfig<false, 1, 1, 4, 4, false> k32x32{{6.24f, 1.37f, 1.81f}};
+
+template <int EPI>
+unsigned go(const GemmArgs& a) {
+  return launch_cheapest<EPI>(a, k256x256, k256x128, k128x192, k128x128, k128x96, k64x128, k64x96, k64x64, k32x64,
+                              k32x32);
+}
+
+}  // namespace
+
+unsigned launch_gemm_tile_bf16(int epi, const GemmArgs& a) {
+  switch (epi) {
+    case kEpiBf16: return go<kEpiBf16>(a);
+    case kEpiF32: return go<kEpiF32>(a);
+    default: return go<kEpiResidual>(a);
+  }
+}
+
+}  // namespace g4
