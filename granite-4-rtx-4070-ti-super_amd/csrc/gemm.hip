@@ -815,6 +815,19 @@ unsigned gemm_grid(long long tiles, int cap) {
   return static_cast<unsigned>(g > 0 ? g : 1);
 }
 
+// Whether M <= kSkinnyMaxM rows take the skinny kernel rather than a tile: it
+// streams the weights best while its 16-column workgroups are at most one per
+// CU (K = 12800 down, 8 rows, us: skinny 12.5, tile 14.6; bf16 O 7.4 / 9.1), but
+// re-reads all activations in each, which past that costs more than the
+// tile's staging (FP8 / bf16 A q|k|v, 1.5 per CU: 2 rows 7.3 / 8.9 against 7.4 /
+// 9.7, 4 rows 8.3 / 9.9 against 7.3 / 9.7; 12800 columns, 3.1 per CU: 1 row
+// FP8 25.6 against 24.5, 16 rows bf16 25.6 against 14.2).
+bool skinny_rows(int M, int ncols) {
+  if (M > kSkinnyMaxM) return false;
+  const int ntile = (ncols + 15) / 16;
+  return ntile <= kCUs || (ntile <= 2 * kCUs && M < 4);
+}
+
 }  // namespace
 
 // One skinny GEMM (M <= 16) over a weight block of three row segments
@@ -848,6 +861,8 @@ int gemm_rows_split(bool fp8, const void* A, int lda, const float* a_scale, cons
     a.seg_out[i] = out[i];
     a.seg_ld[i] = ld[i];
   }
+  // The skinny kernel whatever the width: each output is the same sum as in a
+  // call per segment, whose narrower outputs take it too.
   if (fp8) launch_skinny<true, kEpiBf16>(a, INT_MAX);
   else launch_skinny<false, kEpiBf16>(a, INT_MAX);
   return launch_status("gemm_rows_split");
@@ -904,7 +919,7 @@ int granite4_gemm_fp8(int out, const uint8_t* A, int lda, const float* d_a_scale
     else if (deep == 3) go(gemm_fp8_kernel<E, 64, 3>, gemm_grid<E, 64, 3>(tiles, INT_MAX));
     else go(gemm_fp8_kernel<E, 64>, gemm_grid<E, 64>(tiles, INT_MAX));
   };
-  if (M > kSkinnyMaxM && launch_gemm_tile_fp8(out, a) != 0) return launch_status("granite4_gemm_fp8");
+  if (!skinny_rows(M, N) && launch_gemm_tile_fp8(out, a) != 0) return launch_status("granite4_gemm_fp8");
   switch (out) {
     case GRANITE4_GEMM_BF16: run(std::integral_constant<int, kEpiBf16>{}); break;
     case GRANITE4_GEMM_F32: run(std::integral_constant<int, kEpiF32>{}); break;
@@ -955,13 +970,13 @@ int granite4_prefill_gemm(int out, const uint16_t* A, int lda, const uint8_t* W,
     a.xcd_order = gemm_xcd_order(a.mt, gu);
     return gu;
   };
+  if (!skinny_rows(M, N) && launch_gemm_tile_bf16(out, a) != 0) return launch_status("granite4_prefill_gemm");
   if (M <= kSkinnyMaxM) {
     if (out == GRANITE4_GEMM_BF16) launch_skinny<false, kEpiBf16>(a, INT_MAX);
     else if (out == GRANITE4_GEMM_F32) launch_skinny<false, kEpiF32>(a, INT_MAX);
     else launch_skinny<false, kEpiResidual>(a, INT_MAX);
     return launch_status("granite4_prefill_gemm");
   }
-  if (launch_gemm_tile_bf16(out, a) != 0) return launch_status("granite4_prefill_gemm");
   switch (out) {
     case GRANITE4_GEMM_BF16:
       hipLaunchKernelGGL(gemm_bf16w_kernel<kEpiBf16>,
@@ -1024,10 +1039,10 @@ int granite4_gemm_fp8_swiglu(const uint8_t* A, int lda, const float* d_a_scale,
   a.vec_out = true;
   a.partials = work_partials(d_work);
   const long long tiles = static_cast<long long>(a.mt) * a.nt;
-  unsigned grid;
-  if (M <= kSkinnyMaxM) {
+  unsigned grid = skinny_rows(M, I) ? 0 : launch_gemm_tile_fp8(kEpiSwiglu, a);
+  if (grid == 0 && M <= kSkinnyMaxM) {
     grid = launch_skinny<true, kEpiSwiglu>(a, kMaxPartials);
-  } else if ((grid = launch_gemm_tile_fp8(kEpiSwiglu, a)) == 0) {
+  } else if (grid == 0) {
     grid = gemm_grid<kEpiSwiglu>(tiles, kMaxPartials);
     a.xcd_order = gemm_xcd_order(a.mt, grid);
     hipLaunchKernelGGL(gemm_fp8_kernel<kEpiSwiglu>, grid, 256, 0, stream(), a);

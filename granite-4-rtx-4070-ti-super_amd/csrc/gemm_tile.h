@@ -563,15 +563,7 @@ __global__ __launch_bounds__(256 * KS) __attribute__((amdgpu_waves_per_eu(KS, KS
           for (int e = 0; e < 4; ++e)
             amax = fmaxf(amax, fmaxf(lo_bf16(w[e] & 0x7fff7fffu), hi_bf16(w[e] & 0x7fff7fffu)));
         }
-        uint16_t* dst = ep.out_bf16 + off;
-        if (EPI == kEpiBf16 && a.seg_out[0] != nullptr) {  // an output per segment (bounds multiples of 8)
-          const int sg = n < ep.seg1 ? 0 : (n < ep.seg2 ? 1 : 2);
-          const int at = n - (sg == 0 ? 0 : (sg == 1 ? ep.seg1 : ep.seg2));
-          dst = (sg == 0 ? a.seg_out[0] : sg == 1 ? a.seg_out[1] : a.seg_out[2]) +
-                static_cast<size_t>(m0 + wm * 16 * FM + 16 * b + r) *
-                    (sg == 0 ? a.seg_ld[0] : sg == 1 ? a.seg_ld[1] : a.seg_ld[2]) + at;
-        }
-        *reinterpret_cast<uint4*>(dst) = make_uint4(w[0], w[1], w[2], w[3]);
+        *reinterpret_cast<uint4*>(ep.out_bf16 + off) = make_uint4(w[0], w[1], w[2], w[3]);
       }
       tile_reads_wait();  // the block's reads are done before the next one's writes
     }
