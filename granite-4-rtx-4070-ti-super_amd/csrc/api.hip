@@ -71,6 +71,53 @@ int resident_blocks(const void* kernel, int threads) {
 }
 
 namespace {
+// The current device's scratch pool (stream_scratch), made at its first use;
+// nullptr where it cannot be made.
+hipMemPool_t scratch_pool() {
+  static std::mutex mu;
+  static std::map<int, hipMemPool_t> pools;
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess) return nullptr;
+  std::lock_guard<std::mutex> lock(mu);
+  const auto it = pools.find(dev);
+  if (it != pools.end()) return it->second;
+  hipMemPool_t pool = nullptr;
+  hipMemPoolProps props{};
+  props.allocType = hipMemAllocationTypePinned;
+  props.location.type = hipMemLocationTypeDevice;
+  props.location.id = dev;
+  uint64_t keep = 64u << 20;
+  if (hipMemPoolCreate(&pool, &props) != hipSuccess) pool = nullptr;
+  else if (hipMemPoolSetAttribute(pool, hipMemPoolAttrReleaseThreshold, &keep) != hipSuccess) {
+    (void)hipMemPoolDestroy(pool);
+    pool = nullptr;
+  }
+  (void)hipGetLastError();
+  pools[dev] = pool;
+  return pool;
+}
+}  // namespace
+
+void* stream_scratch(size_t bytes, hipStream_t st) {
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(st, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone) {
+    (void)hipGetLastError();
+    return nullptr;
+  }
+  const hipMemPool_t pool = scratch_pool();
+  void* p = nullptr;
+  if (pool == nullptr || hipMallocFromPoolAsync(&p, bytes, pool, st) != hipSuccess) {
+    (void)hipGetLastError();
+    return nullptr;
+  }
+  return p;
+}
+
+void stream_scratch_done(void* p, hipStream_t st) {
+  if (hipFreeAsync(p, st) != hipSuccess) (void)hipGetLastError();
+}
+
+namespace {
 
 // cos / sin of pos * theta^(-2i/d), evaluated in double and rounded to f32
 // (kernel_math.h:191-206).

@@ -121,6 +121,22 @@ __device__ __forceinline__ bf16x8_t as_bf16x8(uint32_t a, uint32_t b, uint32_t c
   return __builtin_bit_cast(bf16x8_t, u);
 }
 
+// Maximum / sum over the lanes l, l ^ 16, l ^ 32, l ^ 48 (the four lanes of one
+// query column), by row swaps within the vector unit: __shfl_xor goes through
+// the LDS, two dependent round trips per tile.
+__device__ __forceinline__ float col_max4(float x) {
+  const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  const float m = fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1]));
+  const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(m), __float_as_uint(m), false, false);
+  return fmaxf(__uint_as_float(b[0]), __uint_as_float(b[1]));
+}
+__device__ __forceinline__ float col_sum4(float x) {
+  const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  const float m = __uint_as_float(a[0]) + __uint_as_float(a[1]);
+  const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(m), __float_as_uint(m), false, false);
+  return __uint_as_float(b[0]) + __uint_as_float(b[1]);
+}
+
 constexpr float kLog2E = 1.44269504088896341f;
 
 // Exact bf16 pair of two small integers (|x| <= 127).
@@ -865,8 +881,7 @@ void attn_split_kernel(AttnArgs a) {
     for (int mb = 0; mb < 4; ++mb)
 #pragma unroll
       for (int i = 0; i < 4; ++i) mx = fmaxf(mx, sv[mb][i]);
-    mx = fmaxf(mx, __shfl_xor(mx, 16));
-    mx = fmaxf(mx, __shfl_xor(mx, 32));
+    mx = col_max4(mx);
     const float alpha = mx == -INFINITY ? 1.0f : __expf(m - mx);
     m = mx;
     l *= alpha;
@@ -916,8 +931,7 @@ void attn_split_kernel(AttnArgs a) {
     wave_lds_sync();  // this tile's LDS reads are done before the next tile's writes
   }
   // l: sum over the four lanes of this query column.
-  l += __shfl_xor(l, 16);
-  l += __shfl_xor(l, 32);
+  l = col_sum4(l);
 
   // Merge the block's kAttnWaves splits (the combine's formula over these
   // splits): per query column, M = max m_w, w_w = exp(m_w - M), then one
@@ -1083,6 +1097,11 @@ struct PrefillArgs {
   int Hq, stride, rows, base, window;
   const int* d_pt;
   uint16_t* out;      // [rows][Hq][128]
+  // Key splits over workgroups (gridDim.z = nsp > 1): split z of a (row, query
+  // head) leaves its (m, l) and unscaled sums here for the combine launch.
+  int nsp;
+  float2* part_ml;    // [rows][Hq][nsp]
+  float* part_o;      // [rows][Hq][nsp][128]
 };
 
 // Staging of keys [j0, j0 + 64) for all 4 waves, pipelined: a tile's raw
@@ -1326,8 +1345,14 @@ __global__ __launch_bounds__(W * 64) void attn_prefill_kernel(PrefillArgs a) {
     my_lo[cb] = a.window > 0 ? max(0, my_pos[cb] + 1 - a.window) : 0;
   }
   const int last = min(p0 + kPos, a.rows) - 1;
-  const int kv_end = min(a.base + last + 1, a.stride);
-  const int j_first = a.window > 0 ? (max(0, a.base + p0 + 1 - a.window) / kTile) * kTile : 0;
+  int kv_end = min(a.base + last + 1, a.stride);
+  int j_first = a.window > 0 ? (max(0, a.base + p0 + 1 - a.window) / kTile) * kTile : 0;
+  if (a.nsp > 1) {  // this split's tiles
+    const long long tiles = max(kv_end - j_first + kTile - 1, 0) / kTile;
+    const int t0 = static_cast<int>(tiles * blockIdx.z / a.nsp), t1 = static_cast<int>(tiles * (blockIdx.z + 1) / a.nsp);
+    kv_end = min(kv_end, j_first + t1 * kTile);
+    j_first += t0 * kTile;
+  }
 
   bf16x8_t qb[CB][4];
 #pragma unroll
@@ -1442,36 +1467,45 @@ __global__ __launch_bounds__(W * 64) void attn_prefill_kernel(PrefillArgs a) {
           }
         }
       }
-      // Online softmax per column block (e holds the logits until here).
+      // Online softmax (e holds the logits until here): every column block's
+      // maximum first, then one wave-uniform branch for all of them.
+      float mx[CB];
+      bool moved = false;
 #pragma unroll
       for (int cb = 0; cb < CB; ++cb) {
-        float mx = m[cb];
+        mx[cb] = m[cb];
 #pragma unroll
         for (int mb = 0; mb < 4; ++mb)
 #pragma unroll
-          for (int i = 0; i < 4; ++i) mx = fmaxf(mx, e[cb][mb][i]);
-        mx = fmaxf(mx, __shfl_xor(mx, 16));
-        mx = fmaxf(mx, __shfl_xor(mx, 32));
-        // Where no column's maximum moved, the rescale factor is exactly 1:
-        // skip the multiply of o and l (a wave-uniform branch).
-        if (__any(mx != m[cb])) {
-          const float alpha = mx == -INFINITY ? 1.0f : __expf(m[cb] - mx);
-          m[cb] = mx;
+          for (int i = 0; i < 4; ++i) mx[cb] = fmaxf(mx[cb], e[cb][mb][i]);
+        mx[cb] = col_max4(mx[cb]);
+        moved = moved || mx[cb] != m[cb];
+      }
+      // Where no column's maximum moved, every rescale factor is exactly 1:
+      // skip the multiply of o and l.
+      if (__any(moved)) {
+#pragma unroll
+        for (int cb = 0; cb < CB; ++cb) {
+          const float alpha = mx[cb] == -INFINITY ? 1.0f : __expf(m[cb] - mx[cb]);
+          m[cb] = mx[cb];
           l[cb] *= alpha;
 #pragma unroll
           for (int nb = 0; nb < 8; ++nb) o[cb][nb] *= alpha;
         }
+      }
+#pragma unroll
+      for (int cb = 0; cb < CB; ++cb) {
         // exp(e - mx) as exp2(e log2(e) - mx log2(e)): one FMA feeds the
         // hardware exponential instead of a subtraction and a multiply (the
         // argument's error is the rounding of mx log2(e), of the same order as
         // that of (e - mx) log2(e)); T=8192 K5V4 13.63 -> 13.18 ms.
-        const float nml = -mx * kLog2E;
+        const float nml = -mx[cb] * kLog2E;
 #pragma unroll
         for (int mb = 0; mb < 4; ++mb)
 #pragma unroll
           for (int i = 0; i < 4; ++i) {
             const float p = __builtin_amdgcn_exp2f(fmaf(e[cb][mb][i], kLog2E, nml));
-            if constexpr (kMask) e[cb][mb][i] = mx == -INFINITY ? 0.0f : p;
+            if constexpr (kMask) e[cb][mb][i] = mx[cb] == -INFINITY ? 0.0f : p;
             else e[cb][mb][i] = p;
             l[cb] += e[cb][mb][i];
           }
@@ -1553,6 +1587,7 @@ __global__ __launch_bounds__(W * 64) void attn_prefill_kernel(PrefillArgs a) {
       const float mm = fmaxf(m[cb], m1);
       const float a0 = m[cb] == -INFINITY ? 0.0f : __expf(m[cb] - mm);
       const float a1 = m1 == -INFINITY ? 0.0f : __expf(m1 - mm);
+      m[cb] = mm;
       l[cb] = l[cb] * a0 + l1 * a1;
 #pragma unroll
       for (int nb = 0; nb < 8; ++nb) o[cb][nb] = o[cb][nb] * a0 + xo[(cb * 8 + nb) * 64] * a1;
@@ -1560,10 +1595,16 @@ __global__ __launch_bounds__(W * 64) void attn_prefill_kernel(PrefillArgs a) {
   }
 #pragma unroll
   for (int cb = 0; cb < CB; ++cb) {
-    float lt = l[cb];
-    lt += __shfl_xor(lt, 16);
-    lt += __shfl_xor(lt, 32);
+    const float lt = col_sum4(l[cb]);
     if (!live[cb]) continue;
+    if (a.nsp > 1) {
+      const size_t at = (static_cast<size_t>(r[cb]) * a.Hq + hq) * a.nsp + blockIdx.z;
+      if (g == 0) a.part_ml[at] = make_float2(m[cb], lt);
+      float* po = a.part_o + at * kHd + 4 * g;
+#pragma unroll
+      for (int nb = 0; nb < 8; ++nb) *reinterpret_cast<f32x4_t*>(po + 16 * nb) = o[cb][nb];
+      continue;
+    }
     const float inv = 1.0f / lt;
     uint16_t* dst = a.out + (static_cast<size_t>(r[cb]) * a.Hq + hq) * kHd + 4 * g;
 #pragma unroll
@@ -1572,6 +1613,41 @@ __global__ __launch_bounds__(W * 64) void attn_prefill_kernel(PrefillArgs a) {
           u32x2_t{pack_bf16_hw(o[cb][nb][0] * inv, o[cb][nb][1] * inv),
                   pack_bf16_hw(o[cb][nb][2] * inv, o[cb][nb][3] * inv)};
   }
+}
+
+// The key splits of one (row, query head) combined by one wave, in split
+// order: M = max m_z, w_z = exp(m_z - M) (0 for a split without keys of the
+// row), out = bf16(sum o_z w_z * (1 / sum l_z w_z)). Lane z holds split z's
+// (m, l) (at most 64); each lane owns two dims.
+__global__ __launch_bounds__(256) void attn_prefill_combine_kernel(PrefillArgs a) {
+  const int lane = threadIdx.x & 63;
+  const size_t rh = static_cast<size_t>(blockIdx.x) * 4 + (threadIdx.x >> 6);
+  if (rh >= static_cast<size_t>(a.rows) * a.Hq) return;
+  const float* po = a.part_o + rh * a.nsp * kHd + 2 * lane;
+  const float2 ml = a.part_ml[rh * a.nsp + min(lane, a.nsp - 1)];
+  const float mj = lane < a.nsp ? ml.x : -INFINITY;
+  float M = mj;
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) M = fmaxf(M, __shfl_xor(M, o));
+  const float wj = mj == -INFINITY ? 0.0f : __expf(mj - M);
+  float L = 0.0f, acc0 = 0.0f, acc1 = 0.0f;
+  constexpr int kChunk = 8;
+  for (int c = 0; c < a.nsp; c += kChunk) {
+    float2 ov[kChunk];
+#pragma unroll
+    for (int j = 0; j < kChunk; ++j)
+      ov[j] = *reinterpret_cast<const float2*>(po + static_cast<size_t>(min(c + j, a.nsp - 1)) * kHd);
+#pragma unroll
+    for (int j = 0; j < kChunk; ++j) {
+      if (c + j >= a.nsp) break;
+      const float w = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(wj), c + j));
+      L += __int_as_float(__builtin_amdgcn_readlane(__float_as_int(ml.y), c + j)) * w;
+      acc0 += ov[j].x * w;
+      acc1 += ov[j].y * w;
+    }
+  }
+  const float inv = 1.0f / L;
+  *reinterpret_cast<uint32_t*>(a.out + rh * kHd + 2 * lane) = pack_bf16_hw(acc0 * inv, acc1 * inv);
 }
 
 }  // namespace
@@ -1667,19 +1743,62 @@ void launch_prefill_w(const PrefillArgs& a, int group, dim3 grid, hipStream_t st
   }
 }
 
-// 8-wave workgroups of 64 positions (CB = 2) or 32 (CB = 1) where they give
-// every CU one, else 16-position workgroups for twice the workgroups: 8 waves
-// splitting the keys between two 4-wave groups.
+// How a prefill call runs: its workgroup form and its key splits.
+struct PrefillPlan {
+  enum Form { k64, k32, k16x2 } form;  // positions per workgroup (k16x2: keys split inside it)
+  int nsp;                             // key splits over workgroups
+};
+constexpr size_t kPrefillSplitBytes = 48u << 20;  // partials of one call at most
+constexpr int kPrefillMaxSplits = 64;
+
+size_t prefill_split_bytes(int rows, int Hq, int nsp) {
+  return static_cast<size_t>(rows) * Hq * nsp * (kHd + 2) * sizeof(float);
+}
+
+// Without key splits: 8-wave workgroups of 64 positions (CB = 2) or 32 (CB = 1)
+// where they give every CU one, else 16-position workgroups for twice the
+// workgroups: 8 waves splitting the keys between two 4-wave groups.
+//
+// A short chunk at the end of a long context (a conversation's next turn) has
+// few workgroups, each walking the whole context: 17 rows at 50000 took 1.17
+// ms on 16 CUs. There the keys are split over workgroups too, and a second
+// launch combines the partials. The plan is the one with the least predicted
+// time, from a tile's time in each form (measured, us: 64 positions 3.5, 32
+// positions 2.2, 16 positions 3.1 per two tiles, a workgroup per CU) and the
+// splits' cost (a launch, and each partial written and read at 4 TB/s). A
+// split holds at least 4 tiles.
+PrefillPlan prefill_plan(int rows, int base, int window, int Hk, bool may_split) {
+  const auto blocks = [&](int pos) { return static_cast<long long>((rows + pos - 1) / pos) * Hk; };
+  PrefillPlan p{blocks(64) >= kCUs ? PrefillPlan::k64 : blocks(32) >= kCUs ? PrefillPlan::k32 : PrefillPlan::k16x2, 1};
+  if (!may_split || p.form == PrefillPlan::k64) return p;
+  const int span = window > 0 ? (window + rows < base + rows ? window + rows : base + rows) : base + rows;
+  const double tiles = (span + kTile - 1) / kTile;  // the last block's
+  const double per_tile[] = {3.5, 2.2, 1.55};
+  const auto rounds = [](double wgs) { return static_cast<double>((static_cast<long long>(wgs) + kCUs - 1) / kCUs); };
+  double best = p.form == PrefillPlan::k32 ? rounds(static_cast<double>(blocks(32))) * tiles * per_tile[1]
+                                           : rounds(static_cast<double>(blocks(16))) * tiles * per_tile[2];
+  for (const auto form : {PrefillPlan::k64, PrefillPlan::k16x2}) {
+    const int pos = form == PrefillPlan::k64 ? 64 : 16;
+    for (int nsp = 2; nsp <= kPrefillMaxSplits && nsp * 4 <= tiles; ++nsp) {
+      const double bytes = static_cast<double>(prefill_split_bytes(rows, 4 * Hk, nsp));
+      if (bytes > static_cast<double>(kPrefillSplitBytes)) break;
+      const double steps = std::ceil(tiles / nsp);
+      const double t = rounds(static_cast<double>(blocks(pos)) * nsp) * steps * per_tile[form] + 6.0 + 2.0 * bytes / 4e6;
+      if (t < 0.95 * best) best = t, p = PrefillPlan{form, nsp};
+    }
+  }
+  return p;
+}
+
 template <int BITS>
-void launch_prefill_bits(const PrefillArgs& a, int group, int Hk, hipStream_t st) {
-  const long long blocks64 = static_cast<long long>((a.rows + 63) / 64) * Hk;
-  const long long blocks32 = static_cast<long long>((a.rows + 31) / 32) * Hk;
-  if (blocks64 >= kCUs) {
-    launch_prefill_w<BITS, 8, 1, 2>(a, group, dim3((a.rows + 63) / 64, Hk), st);
-  } else if (blocks32 >= kCUs) {
-    launch_prefill_w<BITS, 8, 1, 1>(a, group, dim3((a.rows + 31) / 32, Hk), st);
+void launch_prefill_bits(const PrefillArgs& a, int group, int Hk, PrefillPlan::Form form, hipStream_t st) {
+  const unsigned z = static_cast<unsigned>(a.nsp);
+  if (form == PrefillPlan::k64) {
+    launch_prefill_w<BITS, 8, 1, 2>(a, group, dim3((a.rows + 63) / 64, Hk, z), st);
+  } else if (form == PrefillPlan::k32) {
+    launch_prefill_w<BITS, 8, 1, 1>(a, group, dim3((a.rows + 31) / 32, Hk, z), st);
   } else {
-    launch_prefill_w<BITS, 8, 2, 1>(a, group, dim3((a.rows + 15) / 16, Hk), st);
+    launch_prefill_w<BITS, 8, 2, 1>(a, group, dim3((a.rows + 15) / 16, Hk, z), st);
   }
 }
 
@@ -1719,11 +1838,25 @@ int granite4_prefill_attn(const uint16_t* q_rot, int rows, int Hq, int Hk, int d
   a.d_pt = d_pt;
   a.out = out;
   const hipStream_t st = stream();
+  PrefillPlan plan = prefill_plan(rows, base_pos, window, Hk, true);
+  void* scratch = nullptr;
+  if (plan.nsp > 1) {
+    scratch = stream_scratch(prefill_split_bytes(rows, Hq, plan.nsp), st);
+    if (scratch == nullptr) plan = prefill_plan(rows, base_pos, window, Hk, false);  // under capture
+  }
+  a.nsp = plan.nsp;
+  a.part_o = static_cast<float*>(scratch);
+  a.part_ml = reinterpret_cast<float2*>(a.part_o + static_cast<size_t>(rows) * Hq * plan.nsp * kHd);
   switch (bits) {
-    case 16: launch_prefill_bits<16>(a, group, Hk, st); break;
-    case 8: launch_prefill_bits<8>(a, group, Hk, st); break;
-    case 4: launch_prefill_bits<4>(a, group, Hk, st); break;
-    default: launch_prefill_bits<5>(a, group, Hk, st); break;
+    case 16: launch_prefill_bits<16>(a, group, Hk, plan.form, st); break;
+    case 8: launch_prefill_bits<8>(a, group, Hk, plan.form, st); break;
+    case 4: launch_prefill_bits<4>(a, group, Hk, plan.form, st); break;
+    default: launch_prefill_bits<5>(a, group, Hk, plan.form, st); break;
+  }
+  if (scratch != nullptr) {
+    const long long rh = static_cast<long long>(rows) * Hq;
+    hipLaunchKernelGGL(attn_prefill_combine_kernel, dim3(static_cast<unsigned>((rh + 3) / 4)), 256, 0, st, a);
+    stream_scratch_done(scratch, st);
   }
   return launch_status("granite4_prefill_attn");
 }

@@ -72,6 +72,15 @@ hipStream_t stream();
 // G4_CUDA_CHECK: message on stderr, -1 to the caller.
 int launch_status(const char* what);
 
+// Device memory for one call's launches on `st`, ordered on it: from a pool of
+// the library's own per device, which keeps at most 64 MB between calls and
+// gives the rest back. nullptr while `st` is being captured (a graph may run on
+// another stream and at any time) or where the allocation fails; the caller
+// then takes a form that needs none. stream_scratch_done returns it after the
+// last launch that uses it.
+void* stream_scratch(size_t bytes, hipStream_t st);
+void stream_scratch_done(void* p, hipStream_t st);
+
 // How many workgroups of `threads` threads of `kernel` the current device
 // holds at once (occupancy per CU x CUs); 0 if the query fails. The
 // single-launch FP8 forms launch at most this many, so that every workgroup

@@ -26,8 +26,9 @@
 //   act codes, s' = SwiGLU(GEMM_fp8(codes, Wg|Wu)) -> FP8   gemm_fp8_swiglu
 //   hidden = bf16(hidden + rs * GEMM_fp8(act codes, s', Wd)) gemm_fp8, kResidual
 // Every launch is one of the library's entry points on the calling thread's
-// stream, so a step equals those calls one by one. Nothing is allocated and
-// nothing synchronises: the calls can be captured in a HIP graph. Every
+// stream, so a step equals those calls one by one. Nothing synchronises, and
+// nothing is allocated but the prefill attention's stream-ordered scratch
+// (none under capture): the calls can be captured in a HIP graph. Every
 // argument is checked before the first launch, so a call either launches
 // nothing (-1) or the whole sequence.
 #include "g4_common.h"

@@ -448,6 +448,12 @@ int granite4_prefill_attention(const uint16_t* q_rot, const uint16_t* cache_k,
                                const uint8_t* cache_k4, const uint8_t* cache_v4, int int4,
                                const int* d_pt, int k5, int window);
 
+/* A chunk too short to give every CU a workgroup at the end of a long context
+ * splits its keys over workgroups: the partials take scratch from a
+ * stream-ordered pool of the library's own (at most 48 MB per call; the pool
+ * keeps at most 64 MB per device between calls), and a second launch combines
+ * them. Under stream capture no scratch is taken and the keys are not split;
+ * the two agree to the rounding of the bf16 probabilities. */
 /* granite4_prefill_attention for every pool format of this library (bits 16
  * / 8 / 4 / 5, group 32 / 64 / 128 scales; groups of 32 / 64 read as
  * granite4_attn_paged reads them). New entry point. */

@@ -590,3 +590,35 @@ def test_attn_combine_in_split_launch_graph_replays():
     finally:
         L.set_attn_combine_mode(prev)
         L.use_stream()
+
+
+# A short chunk at the end of a long context: the keys are split over
+# workgroups (16- and 64-position forms) and combined by a second launch.
+@pytest.mark.parametrize("rows,bits,group,window", [(17, 8, 128, 0), (16, 16, 128, 0), (33, 5, 32, 0),
+                                                    (64, 4, 64, 2000), (130, 8, 64, 0)])
+def test_prefill_attn_key_splits(rows, bits, group, window):
+    note(f"prefill attn key splits rows={rows} bits={bits} group={group} window={window}")
+    base = 3001
+    pages = (base + rows + 15) // 16 + 2
+    stride = 16 * pages
+    ck, cv, ks, vs = make_cache(bits, group, stride, 0xA4 + bits)
+    rng = np.random.default_rng(bits + rows)
+    pt = ol.row_table(rng.permutation(pages).astype(np.int32), stride)
+    q = ol.normal_bf16(0xA5, 0.0, 1.0, rows * HQ * D).reshape(rows, HQ * D)
+    want = ol.prefill_attn(q, ck, cv, ks, vs, bits, group, stride, base, pt=pt, window=window,
+                           scale=1.0 / 16, Hk=HK)
+    got = run_prefill(q, ck, cv, ks, vs, bits, group, stride, base, d_pt=dev(pt), window=window)
+    check(got, want, vmax(cv, vs, bits), f"key splits rows {rows}")
+    # Under capture no scratch is taken: the unsplit form, replayed.
+    args = [dev(q), dev(ck), dev(cv), None if ks is None else dev(ks), None if vs is None else dev(vs),
+            dev(pt), torch.zeros((rows, HQ * D), dtype=torch.int16, device="cuda")]
+    graph, cap = torch.cuda.CUDAGraph(), torch.cuda.Stream()
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graph, stream=cap):
+        L.use_stream(cap)
+        L.call("granite4_prefill_attn", args[0], rows, HQ, HK, D, 1.0 / 16, *args[1:5], bits, group,
+               stride, base, args[5], window, args[6])
+    L.use_stream()
+    for _ in range(2):
+        graph.replay()
+        check(host(args[6]).view(np.uint16), want, vmax(cv, vs, bits), f"captured rows {rows}")
