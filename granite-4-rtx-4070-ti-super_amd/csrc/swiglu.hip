@@ -182,12 +182,18 @@ __global__ __launch_bounds__(kBlock) void encode_bf16_kernel(SwArgs a) {
 // VGPRs; the workgroups agree on max |act| with one grid synchronisation and
 // encode what they hold. HBM traffic is the algorithmic 4 B read + 1 B
 // written per element (+2 B with the optional bf16 act), against 9 B for
-// the two-launch form, and one launch instead of two.
+// the two-launch form, and one launch instead of two. Two instances: up to 4
+// vectors per lane, and up to 8 (all their loads in flight at once, still
+// four waves per SIMD), which ends at 1310 rows of 12800 on a full grid.
+// Between 656 and 1310 rows the held form below took its place before, whose
+// two loads in flight per lane leave a short sweep waiting on memory (and
+// which then loaded held vectors that no lane has): 656 rows 39.2 -> 16.3 us,
+// 1024 40.6 -> 19.3, 1300 42.8 -> 22.0.
 constexpr int kFusedThreads = kBlock;
 static_assert(kFusedThreads == kSyncThreads && kBlock == kSyncThreads, "grid_max assumes kSyncThreads-thread workgroups");
-constexpr int kFusedVpt = 4;
 
-__global__ __launch_bounds__(kFusedThreads) void swiglu_fp8_fused_kernel(SwArgs a, GridSync gs) {
+template <int kFusedVpt>
+__global__ __launch_bounds__(kFusedThreads) __attribute__((amdgpu_waves_per_eu(4))) void swiglu_fp8_fused_kernel(SwArgs a, GridSync gs) {
   // Every argument of the first loads fetched in one scalar round trip.
   asm volatile("" ::"s"(a.gu), "s"(a.rows), "s"(a.I), "s"(a.inv_nv), "s"(a.act), "s"(a.codes),
                "s"(gs.gen), "s"(gs.slots), "s"(gs.result), "s"(gs.blocks));
@@ -250,9 +256,10 @@ __global__ __launch_bounds__(kFusedThreads) void swiglu_fp8_fused_kernel(SwArgs 
 // where the grid allows (up to kMaxPartials workgroups, the slot count):
 // measured against 1024-thread workgroups on one per CU, T=512 14.0 vs
 // 14.8 us and T=8 5.9 vs 7.4 us.
+template <int kFusedVpt>
 unsigned fused_grid(long long vectors) {
   if (fp8_launch_mode() == 1) return 0;
-  const int resident = resident_blocks(reinterpret_cast<const void*>(swiglu_fp8_fused_kernel),
+  const int resident = resident_blocks(reinterpret_cast<const void*>(swiglu_fp8_fused_kernel<kFusedVpt>),
                                        kFusedThreads);
   const int cap = resident < kMaxPartials ? resident : kMaxPartials;
   const long long per_block = static_cast<long long>(kFusedThreads) * kFusedVpt;
@@ -273,7 +280,10 @@ unsigned fused_grid(long long vectors) {
 // (the oldest otherwise runs ahead and the youngest ends the launch late).
 // HBM traffic per element: 4 B read + 1 B written
 // + 4 B re-read for the streamed fraction only (the two-launch form
-// re-reads everything: 9 B).
+// re-reads everything: 9 B). A batch of held vectors that no lane has is
+// skipped, and so is the streamed re-read where nothing is streamed (their
+// clamped loads all fell on the tensor's last line): 1400 rows of 12800
+// 43.7 -> 25.4 us, 2048 46.0 -> 31.4, 4096 56.3 -> 48.7, 8192 unchanged (108).
 // Held vectors per lane (VGPRs, LDS), held loads and streamed loads in
 // flight per lane, waves per SIMD. Measured at T=8192 (µs, one box, four
 // interleaved rounds): (18, 9, 4, 2, 4) 131.9-137.3, (22, 9, 2, 1, 4)
@@ -319,8 +329,10 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kHoldWav
   // Vectors per lane over both parts (held, then streamed), for the issue
   // priority by progress.
   const int per_lane = (total + step - 1) / step;
-#pragma unroll
-  for (int k0 = 0; k0 < kHold; k0 += kHoldBatch) {
+  static_for<(kHold + kHoldBatch - 1) / kHoldBatch>([&](auto bc) {
+    constexpr int k0 = decltype(bc)::value * kHoldBatch;
+    // (no lane has these vectors; clamped loads of them would all hit one line)
+    if (k0 >= per_lane) return;
     wave_priority_by_progress(k0, per_lane);
     GuRaw<false> x[kHoldBatch];
 #pragma unroll
@@ -339,7 +351,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kHoldWav
         s_hold[k >= kHoldR ? k - kHoldR : 0][threadIdx.x] = make_uint4(o[0], o[1], o[2], o[3]);
       }
     }
-  }
+  });
   G4_TRACE_MARK(gs, 1);
   // The streamed rest: max only (cached loads: part is still cached when
   // the second sweep comes back to it).
@@ -406,7 +418,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kHoldWav
           if (vn < total) streamed(xs, vn);
           vn += step;
         }
-        xs = load_gu<false, true>(a, min(vn, total - 1), nv);
+        if (vs - v0 < total) xs = load_gu<false, true>(a, min(vn, total - 1), nv);
       }
     });
     if constexpr (kMix > 0) {
@@ -543,7 +555,8 @@ int granite4_swiglu_fp8(const uint16_t* d_gu, int rows, int I, uint8_t* d_codes,
     return -1;
   }
   const long long vectors = static_cast<long long>(rows) * (I / 8);
-  const unsigned fgrid = fused_grid(vectors);
+  const unsigned fgrid4 = fused_grid<4>(vectors);
+  const unsigned fgrid = fgrid4 != 0 ? fgrid4 : fused_grid<8>(vectors);
   if (fgrid != 0) {
     SwArgs f = sw_args(d_gu, rows, I);
     f.act = d_act;
@@ -551,7 +564,8 @@ int granite4_swiglu_fp8(const uint16_t* d_gu, int rows, int I, uint8_t* d_codes,
     f.scale_out = d_scale;
     const GridSync gs{work_slots(d_work), work_gen(d_work), work_result(d_work),
                       static_cast<int>(fgrid), work_err(d_work), fp8_sync_spin_limit()};
-    launch_grid_sync(swiglu_fp8_fused_kernel, fgrid, kFusedThreads, stream(), f, gs);
+    launch_grid_sync(fgrid4 != 0 ? swiglu_fp8_fused_kernel<4> : swiglu_fp8_fused_kernel<8>, fgrid, kFusedThreads,
+                     stream(), f, gs);
     return launch_status("granite4_swiglu_fp8");
   }
   const unsigned hgrid = hold_grid(vectors);

@@ -828,3 +828,26 @@ def test_fp8_cooperative_launch_mode(op, rows):
     finally:
         L.set_fp8_launch_mode(prev)
     assert L.fp8_sync_status(work) == 0
+
+
+# The held single-launch forms around their bounds on a full grid of 1024
+# workgroups: 4 vectors per lane (655 rows of 12800), 8 (1310 rows), then the
+# form that skips the held vectors no lane has, up to its streamed part (5080
+# rows of 12800 on such a grid). Codes and scale equal the two-launch form's.
+@pytest.mark.parametrize("rows", [655, 656, 1310, 1311, 1400, 2621, 5079, 5081])
+def test_swiglu_fp8_held_vectors_match_two_launches(rows):
+    note(f"swiglu fp8 held vectors rows={rows}")
+    g = torch.Generator(device="cuda")
+    g.manual_seed(rows)
+    gu = torch.randn((rows, 2 * 12800), generator=g, device="cuda").to(torch.bfloat16)
+    work = L.fp8_workspace()
+    got = []
+    for mode in (0, 1):
+        prev = L.set_fp8_launch_mode(mode)
+        codes, scale = L.swiglu_fp8(gu, work)
+        torch.cuda.synchronize()
+        L.set_fp8_launch_mode(prev)
+        got.append((codes, scale))
+    assert L.fp8_sync_status(work) == 0
+    assert torch.equal(got[0][1], got[1][1])
+    assert torch.equal(got[0][0], got[1][0])
