@@ -1303,8 +1303,13 @@ __device__ __forceinline__ void prefill_store(const PrefillRaw<BITS, GROUP, W>& 
 // at the end group 1's (m, l, o) merge into group 0's through LDS
 // (M = max m, each side's o and l scaled by exp(m - M)). Two waves per SIMD
 // where a short prompt gives each CU one 16-position workgroup.
+//
+// Two waves per SIMD, asked for (2, 2) also where a form needs few enough
+// registers for two workgroups on one CU: those share a CU while others stand
+// idle (int8 from position 0: 1000 tokens, 256 workgroups, 41.8 -> 38.6 us,
+// 1500 66.1 -> 55.9).
 template <int BITS, int GROUP, int CB, int W, int KSP = 1>
-__global__ __launch_bounds__(W * 64) void attn_prefill_kernel(PrefillArgs a) {
+__global__ __launch_bounds__(W * 64) __attribute__((amdgpu_waves_per_eu(2, 2))) void attn_prefill_kernel(PrefillArgs a) {
   static_assert(KSP == 1 || (KSP == 2 && W == 8), "key split: two 4-wave groups");
   constexpr int kPrefWaves = W / KSP;  // waves owning positions (and staging a tile)
   constexpr bool kQuant = BITS != 16;
@@ -1408,6 +1413,18 @@ __global__ __launch_bounds__(W * 64) void attn_prefill_kernel(PrefillArgs a) {
   // Both groups run the same number of steps (one barrier each); group 1
   // idles through the last when the tile count is odd.
   const int steps = kv_end > j_first ? (kv_end - j_first + kStep - 1) / kStep : 0;
+  // The query fragments are waited for here: the loop would otherwise wait for
+  // every load in flight at the top of each tile.
+#pragma unroll
+  for (int cb = 0; cb < CB; ++cb)
+#pragma unroll
+    for (int s = 0; s < 4; ++s) asm volatile("" : "+v"(qb[cb][s]));
+  // The second half of the waves (each shares a SIMD with one of the first)
+  // stages the next tile before its own tile's products, the first half after
+  // them: one converts while the other multiplies. T=8192 at 57344, us: K5V4
+  // 10763 -> 9798, int8 9877 -> 9075, bf16 9621 -> 8905 (with the rows' check
+  // in the middle of the logits, below).
+  const bool early = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x)) >= W * 32;
   int buf = 0;
   for (int it = 0; it < steps; ++it, buf ^= 1) {
     const int j0 = jg + it * kStep;
@@ -1415,6 +1432,19 @@ __global__ __launch_bounds__(W * 64) void attn_prefill_kernel(PrefillArgs a) {
       __syncthreads();
       continue;
     }
+    // Stage the group's next tile (its bytes were loaded a tile ago) into its
+    // other buffer, whose last readers passed the previous barrier; then load
+    // the bytes of the tile after it and the page-table entries of the third.
+    const auto stage_next = [&]() __attribute__((always_inline)) {
+      if (j0 + kStep >= kv_end) return;
+      prefill_store<BITS, GROUP, PW>(raw, ks2[gk][buf ^ 1], vs2[gk][buf ^ 1], ksc2[gk][buf ^ 1],
+                                     vsc2[gk][buf ^ 1], valid2[gk][buf ^ 1], a.scale, tst);
+      if (j0 + 2 * kStep >= kv_end) return;
+      prefill_load<BITS, GROUP, PW>(a, kbase, vbase, kscb, vscb, j0 + 2 * kStep, kv_end, ptk, ptv, raw,
+                                    tst);
+      prefill_pt<BITS, GROUP, PW>(a, j0 + 3 * kStep, kv_end, ptk, ptv, tst);
+    };
+    if (early) stage_next();
     const uint16_t* ks = ks2[gk][buf];
     const uint16_t* vs = vs2[gk][buf];
     const float* ksc_l = ksc2[gk][buf];
@@ -1422,24 +1452,29 @@ __global__ __launch_bounds__(W * 64) void attn_prefill_kernel(PrefillArgs a) {
     const unsigned* s_valid = valid2[gk][buf];
     // A tile that every column of this wave sees whole (all keys at or below
     // the wave's first position, at or above its last window start, each with
-    // an arena row) takes the form without the mask.
-    const bool full = wave_live && j0 + kTile - 1 <= wave_pos_min && j0 >= wave_lo_max &&
-                      __all(s_valid[lane] != 0u);
-    auto tile = [&](auto mask_tag) {
-      constexpr bool kMask = decltype(mask_tag)::value;
+    // an arena row) skips the mask. There is one body for both, the mask a
+    // branch over the logits: with a copy of the body for each, the sums o did
+    // not keep their registers across the two (32 moves of register pairs a
+    // tile) and 6 to 17 registers spilled. T=8192 at 57344, us: K5V4 13569 ->
+    // 10576, int8 11663 -> 9655, bf16 13109 -> 9248.
+    unsigned lane_valid = s_valid[lane];
+    {
       float e[CB][4][4];
+      bool all_valid = true;
 #pragma unroll
       for (int mb = 0; mb < 4; ++mb) {
+        if (mb == 2) {  // (read before the products, waited for in their midst)
+          asm volatile("" : "+v"(lane_valid));
+          all_valid = __all(lane_valid != 0u);
+        }
         bf16x8_t ka[4];
 #pragma unroll
         for (int s = 0; s < 4; ++s)
           ka[s] = *reinterpret_cast<const bf16x8_t*>(ks + (16 * mb + n) * kKPitch + 32 * s + 8 * g);
         float ksv[4][kNgrpB];
-        bool kv_ok[4];
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
           const int key = 16 * mb + 4 * g + i;
-          kv_ok[i] = kMask ? s_valid[key] != 0u : true;
 #pragma unroll
           for (int gi = 0; gi < kNgrpB; ++gi) ksv[i][gi] = kQB ? ksc_l[key * kNgrp + gi] : 1.0f;
         }
@@ -1454,18 +1489,26 @@ __global__ __launch_bounds__(W * 64) void attn_prefill_kernel(PrefillArgs a) {
           for (int i = 0; i < 4; ++i) acc[i] = acc[i] * (kQB ? ksv[i][0] : a.scale);
           const uint32_t lg01 = pack_bf16_hw(acc[0], acc[1]);
           const uint32_t lg23 = pack_bf16_hw(acc[2], acc[3]);
-          const float lg[4] = {lo_bf16(lg01), hi_bf16(lg01), lo_bf16(lg23), hi_bf16(lg23)};
+          e[cb][mb][0] = lo_bf16(lg01);
+          e[cb][mb][1] = hi_bf16(lg01);
+          e[cb][mb][2] = lo_bf16(lg23);
+          e[cb][mb][3] = hi_bf16(lg23);
+        }
+      }
+      const bool full = wave_live && j0 + kTile - 1 <= wave_pos_min && j0 >= wave_lo_max && all_valid;
+      if (!full) {
+#pragma unroll
+        for (int mb = 0; mb < 4; ++mb)
 #pragma unroll
           for (int i = 0; i < 4; ++i) {
-            if constexpr (kMask) {
-              const int j = j0 + 16 * mb + 4 * g + i;
-              const bool ok = live[cb] && j <= my_pos[cb] && j >= my_lo[cb] && kv_ok[i];
-              e[cb][mb][i] = ok ? lg[i] : -INFINITY;
-            } else {
-              e[cb][mb][i] = lg[i];
+            const int key = 16 * mb + 4 * g + i, j = j0 + key;
+            const bool kv_ok = s_valid[key] != 0u;
+#pragma unroll
+            for (int cb = 0; cb < CB; ++cb) {
+              const bool ok = live[cb] && j <= my_pos[cb] && j >= my_lo[cb] && kv_ok;
+              e[cb][mb][i] = ok ? e[cb][mb][i] : -INFINITY;
             }
           }
-        }
       }
       // Online softmax (e holds the logits until here): every column block's
       // maximum first, then one wave-uniform branch for all of them.
@@ -1499,14 +1542,13 @@ __global__ __launch_bounds__(W * 64) void attn_prefill_kernel(PrefillArgs a) {
         // hardware exponential instead of a subtraction and a multiply (the
         // argument's error is the rounding of mx log2(e), of the same order as
         // that of (e - mx) log2(e)); T=8192 K5V4 13.63 -> 13.18 ms.
-        const float nml = -mx[cb] * kLog2E;
+        // A column without a key so far has only -inf here: exp2(-inf + 0) = 0.
+        const float nml = mx[cb] == -INFINITY ? 0.0f : -mx[cb] * kLog2E;
 #pragma unroll
         for (int mb = 0; mb < 4; ++mb)
 #pragma unroll
           for (int i = 0; i < 4; ++i) {
-            const float p = __builtin_amdgcn_exp2f(fmaf(e[cb][mb][i], kLog2E, nml));
-            if constexpr (kMask) e[cb][mb][i] = mx[cb] == -INFINITY ? 0.0f : p;
-            else e[cb][mb][i] = p;
+            e[cb][mb][i] = __builtin_amdgcn_exp2f(fmaf(e[cb][mb][i], kLog2E, nml));
             l[cb] += e[cb][mb][i];
           }
       }
@@ -1545,22 +1587,8 @@ __global__ __launch_bounds__(W * 64) void attn_prefill_kernel(PrefillArgs a) {
             o[cb][nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(va, pb[cb][gi], o[cb][nb], 0, 0, 0);
         }
       }
-    };
-    if (full) tile(std::false_type{});
-    else tile(std::true_type{});
-    if (j0 + kStep < kv_end) {
-      // Stage the group's next tile (its bytes were loaded a tile ago) into
-      // its other buffer, whose last readers passed the previous barrier;
-      // then load the bytes of the tile after it and the page-table entries
-      // of the third.
-      prefill_store<BITS, GROUP, PW>(raw, ks2[gk][buf ^ 1], vs2[gk][buf ^ 1], ksc2[gk][buf ^ 1],
-                                     vsc2[gk][buf ^ 1], valid2[gk][buf ^ 1], a.scale, tst);
-      if (j0 + 2 * kStep < kv_end) {
-        prefill_load<BITS, GROUP, PW>(a, kbase, vbase, kscb, vscb, j0 + 2 * kStep, kv_end, ptk,
-                                      ptv, raw, tst);
-        prefill_pt<BITS, GROUP, PW>(a, j0 + 3 * kStep, kv_end, ptk, ptv, tst);
-      }
     }
+    if (!early) stage_next();
     __syncthreads();
   }
   if constexpr (KSP == 2) {
