@@ -44,6 +44,7 @@
 #include "granite4_layerops.h"
 #include "rope_unit.h"
 
+#include <algorithm>
 #include <atomic>
 #include <climits>
 #include <cstdlib>
@@ -1080,8 +1081,7 @@ __global__ __launch_bounds__(kCombineThreads) void attn_combine_kernel(AttnArgs 
 // output is bf16(o * (1 / l)) (prefill_gemm.cu:930-940).
 // ---------------------------------------------------------------------------
 constexpr int kKPitch = kHd + 8;  // K tile pitch (bf16): 272 B, 16 rows on distinct banks
-// Waves per prefill workgroup (template parameter W): 8, or 4 where 8-wave
-// workgroups would not give every CU one. Staging a tile's K / V into LDS is
+// Waves per prefill workgroup (template parameter W): 8. Staging a tile's K / V into LDS is
 // split over all of them, so more waves sharing a tile cost less staging per
 // score; fewer waves per workgroup give short prompts more workgroups.
 // Measured: T=8192 at 57344 K5V4 8 waves 23.6 ms, 4 waves 48.5 ms; T=512
@@ -1749,15 +1749,9 @@ void launch_attn_bits(const AttnArgs& a, int group, dim3 grid, hipStream_t st) {
 }
 
 // Column blocks per wave: CB = 2 (each wave 8 positions x the 4 query heads,
-// 64 positions per 8-wave workgroup) where those workgroups still give every
-// CU one, else CB = 1. Two column blocks halve the staging (code -> bf16
-// conversion, the VALU-heaviest part) per MFMA; with fewer workgroups the
-// occupancy they cost matters more. Measured (8 KV heads, one box, us): int8
-// from position 0, CB = 1 / 2: T=1024 46.3 / 50.5 (CB = 2 there runs the
-// key-split form), 2048 161.9 / 122.8, 4096 462.5 / 444.1, 8192 1475 / 1274;
-// K5V4 group 32 at 57344..: T=2048 4288 / 3482, 4096 8583 / 7102, 8192 18357
-// / 14779. (Before the group-32 tiles were staged dequantised: CB = 1 / 2 / 4
-// at T=512 int8 33.7 / 45.1 / 69.0 us, at T=8192 K5V4 38.2 / 49.2 / 42.2 ms.)
+// 64 positions per 8-wave workgroup) halves the staging (code -> bf16
+// conversion) and the fragment reads per MFMA against CB = 1; prefill_plan
+// takes it where its fewer, longer workgroups keep the CUs as busy.
 
 template <int BITS, int W, int KSP = 1, int CB = 1>
 void launch_prefill_w(const PrefillArgs& a, int group, dim3 grid, hipStream_t st) {
@@ -1783,36 +1777,50 @@ size_t prefill_split_bytes(int rows, int Hq, int nsp) {
   return static_cast<size_t>(rows) * Hq * nsp * (kHd + 2) * sizeof(float);
 }
 
-// Without key splits: 8-wave workgroups of 64 positions (CB = 2) or 32 (CB = 1)
-// where they give every CU one, else 16-position workgroups for twice the
-// workgroups: 8 waves splitting the keys between two 4-wave groups.
+// Three workgroup forms: 8 waves with 64 positions (CB = 2) or 32 (CB = 1), and
+// 16 positions with the keys split between two 4-wave groups. Fewer positions
+// give more workgroups, whose lengths balance better where the causal rows
+// grow from nothing, and cost more per position.
 //
 // A short chunk at the end of a long context (a conversation's next turn) has
 // few workgroups, each walking the whole context: 17 rows at 50000 took 1.17
 // ms on 16 CUs. There the keys are split over workgroups too, and a second
-// launch combines the partials. The plan is the one with the least predicted
-// time, from a tile's time in each form (measured, us: 64 positions 3.5, 32
-// positions 2.2, 16 positions 3.1 per two tiles, a workgroup per CU) and the
-// splits' cost (a launch, and each partial written and read at 4 TB/s). A
-// split holds at least 4 tiles.
+// launch combines the partials. A split holds at least 4 tiles.
+//
+// The plan is the one with the least predicted time: a tile's time in each form
+// (measured, us: 64 positions 2.95, or 2.45 where a CU runs several workgroups
+// in turn, 32 positions 2.1, 16 positions 2.9 per two tiles) times the tiles
+// that the busiest CU runs: the longest workgroup's, or the mean load, or full
+// rounds of the shortest ones (longest first, the CUs even out). Splits add a launch, and each partial
+// written and read at 4 TB/s. Within 9 % of the best of the three forms and up
+// to 16 splits at 20 shapes of 17 to 4096 rows. Against 64 positions wherever
+// those give every CU a workgroup, else 32, else 16 (int8 from 0, us): 1000
+// rows 37.9 -> 31.3, 2000 rows 101.5 -> 76.7, 2500 rows 124 -> 114.
 PrefillPlan prefill_plan(int rows, int base, int window, int Hk, bool may_split) {
-  const auto blocks = [&](int pos) { return static_cast<long long>((rows + pos - 1) / pos) * Hk; };
-  PrefillPlan p{blocks(64) >= kCUs ? PrefillPlan::k64 : blocks(32) >= kCUs ? PrefillPlan::k32 : PrefillPlan::k16x2, 1};
-  if (!may_split || p.form == PrefillPlan::k64) return p;
-  const int span = window > 0 ? (window + rows < base + rows ? window + rows : base + rows) : base + rows;
-  const double tiles = (span + kTile - 1) / kTile;  // the last block's
-  const double per_tile[] = {3.5, 2.2, 1.55};
-  const auto rounds = [](double wgs) { return static_cast<double>((static_cast<long long>(wgs) + kCUs - 1) / kCUs); };
-  double best = p.form == PrefillPlan::k32 ? rounds(static_cast<double>(blocks(32))) * tiles * per_tile[1]
-                                           : rounds(static_cast<double>(blocks(16))) * tiles * per_tile[2];
-  for (const auto form : {PrefillPlan::k64, PrefillPlan::k16x2}) {
-    const int pos = form == PrefillPlan::k64 ? 64 : 16;
-    for (int nsp = 2; nsp <= kPrefillMaxSplits && nsp * 4 <= tiles; ++nsp) {
-      const double bytes = static_cast<double>(prefill_split_bytes(rows, 4 * Hk, nsp));
-      if (bytes > static_cast<double>(kPrefillSplitBytes)) break;
-      const double steps = std::ceil(tiles / nsp);
-      const double t = rounds(static_cast<double>(blocks(pos)) * nsp) * steps * per_tile[form] + 6.0 + 2.0 * bytes / 4e6;
-      if (t < 0.95 * best) best = t, p = PrefillPlan{form, nsp};
+  constexpr int kPositions[] = {64, 32, 16};
+  constexpr double kPerTile[] = {2.95, 2.1, 1.45}, kPerTileInTurn[] = {2.45, 2.1, 1.45};
+  const auto tiles = [&](int pos, int end) {  // of the workgroup whose last position is end - 1
+    const int span = window > 0 && window < end - pos ? window + pos : end;
+    return (span + kTile - 1) / kTile;
+  };
+  PrefillPlan p{PrefillPlan::k64, 1};
+  double best = 0.0;
+  for (const auto form : {PrefillPlan::k64, PrefillPlan::k32, PrefillPlan::k16x2}) {
+    const int pos = kPositions[form];
+    const long long blocks = static_cast<long long>((rows + pos - 1) / pos) * Hk;
+    const int longest = tiles(pos, base + rows), shortest = tiles(pos, base + (rows < pos ? rows : pos));
+    for (int nsp = 1; nsp == 1 || (nsp <= kPrefillMaxSplits && nsp * 4 <= longest); ++nsp) {
+      double extra = 0.0;
+      if (nsp > 1) {
+        const double bytes = static_cast<double>(prefill_split_bytes(rows, 4 * Hk, nsp));
+        if (!may_split || form == PrefillPlan::k32 || bytes > static_cast<double>(kPrefillSplitBytes)) break;
+        extra = 6.0 + 2.0 * bytes / 4e6;
+      }
+      const double wgs = static_cast<double>(blocks) * nsp, top = std::ceil(static_cast<double>(longest) / nsp);
+      const double mean = wgs / kCUs * 0.5 * (longest + shortest) / nsp;
+      const double rounds = std::ceil(wgs / kCUs) * std::ceil(static_cast<double>(shortest) / nsp);
+      const double t = std::max(kPerTile[form] * top, kPerTileInTurn[form] * std::max(mean, rounds)) + extra;
+      if (best == 0.0 || t < 0.95 * best) best = t, p = PrefillPlan{form, nsp};
     }
   }
   return p;

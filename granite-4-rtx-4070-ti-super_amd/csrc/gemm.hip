@@ -19,6 +19,11 @@
 //             the kF32 output without storing it), plus each workgroup's
 //             max |act| for the per-tensor FP8 scale of the encode pass.
 //
+// Three kernels: up to 16 rows the skinny one (skinny_rows), from there on the
+// tile kernel (gemm_tile.h) where K is a multiple of its steps, and the two
+// general ones laid out next for other K (their times at layer shapes, below,
+// are from before the tile kernel took those).
+//
 // Layout: 256-thread workgroups on 128 x 128 output tiles (swiglu: 64 act
 // columns = 64 gate + 64 up weight rows), 4 waves in 2 x 2, each wave 4 x 4
 // v_mfma_f32_16x16x128_f8f6f4 tiles. K advances 128 bytes per stage through

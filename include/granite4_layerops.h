@@ -12,9 +12,10 @@
  *     diagnostic on stderr; outputs are untouched when -1 comes from argument
  *     validation;
  *   - launches are asynchronous on the calling host thread's current stream
- *     (hipStreamPerThread unless granite4_set_stream chose another), never
- *     synchronise and never allocate, so a caller may capture them in a HIP
- *     graph;
+ *     (hipStreamPerThread unless granite4_set_stream chose another) and never
+ *     synchronise, so a caller may capture them in a HIP graph; none allocates,
+ *     except granite4_prefill_attn and its callers, which may take
+ *     stream-ordered scratch outside a capture (said there);
  *   - decode variants read the position from device memory (d_pos).
  *
  * Shapes of the Granite 4.2 8B model: H = 4096, I = 12800, Hq = 32, Hk = 8,
@@ -810,8 +811,9 @@ typedef struct Granite4BatchBuffers {
  * bf16(lm_scale * lm_head . that) [rows][vocab] where given. ops: one of
  * GRANITE4_OPS_*. The FP8 form needs the gate and up weights as one
  * [2I][H] block (wu == wg + I * H). Per layer: 9 launches (bf16; 10 when
- * q, k and v are not one [nqkv][H] block) or 8 (FP8). Asynchronous, no
- * allocation; -1 before any launch on invalid arguments. No reference
+ * q, k and v are not one [nqkv][H] block) or 8 (FP8), and one more where the
+ * attention splits its keys (granite4_prefill_attn, which then takes scratch).
+ * Asynchronous; -1 before any launch on invalid arguments. No reference
  * counterpart as one exported call (the reference's is internal). */
 int granite4_prefill_layers(const Granite4DecodeModel* model, const Granite4BatchBuffers* buffers,
                             const int32_t* d_tokens, int start, int rows, const int* d_pt,

@@ -622,3 +622,26 @@ def test_prefill_attn_key_splits(rows, bits, group, window):
     for _ in range(2):
         graph.replay()
         check(host(args[6]).view(np.uint16), want, vmax(cv, vs, bits), f"captured rows {rows}")
+
+
+# Chunks from position 0, whose workgroups differ most in length: 1000 rows run
+# the 16-position form over two rounds of workgroups, 2000 rows the 32-position
+# one; one KV head leaves CUs for key splits, of which the first rows' shares
+# are empty. The oracle's rows at both ends and in the middle.
+@pytest.mark.parametrize("rows,bits,group,hk", [(1000, 8, 128, HK), (2000, 5, 32, HK), (2000, 16, 128, HK),
+                                                (1000, 8, 64, 1), (1200, 16, 128, 1)])
+def test_prefill_attn_forms_from_zero(rows, bits, group, hk):
+    note(f"prefill attn forms rows={rows} bits={bits} group={group} hk={hk}")
+    pages = (rows + 15) // 16 + 1
+    stride = 16 * pages
+    ck, cv, ks, vs = make_cache(bits, group, stride, 0xB4 + bits)
+    pt = ol.row_table(np.random.default_rng(rows + bits).permutation(pages).astype(np.int32), stride)
+    nq = 4 * hk * D
+    q = ol.normal_bf16(0xB5, 0.0, 1.0, rows * nq).reshape(rows, nq)
+    out = torch.empty((rows, nq), dtype=torch.int16, device="cuda")
+    L.call("granite4_prefill_attn", dev(q), rows, 4 * hk, hk, D, 1.0 / 16, dev(ck), dev(cv),
+           None if ks is None else dev(ks), None if vs is None else dev(vs), bits, group, stride, 0, dev(pt), 0, out)
+    got = host(out).view(np.uint16)
+    for r0, r1 in ((0, 34), (rows // 2 - 9, rows // 2 + 9), (rows - 34, rows)):
+        want = ol.prefill_attn(q[r0:r1], ck, cv, ks, vs, bits, group, stride, r0, pt=pt, scale=1.0 / 16, Hk=hk)
+        check(got[r0:r1], want, vmax(cv, vs, bits), f"rows {r0}..{r1}")
