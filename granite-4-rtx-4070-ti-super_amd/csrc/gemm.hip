@@ -835,12 +835,18 @@ bool skinny_rows(int M, int ncols) {
 
 }  // namespace
 
+// Whether granite4_gemm_fp8 / granite4_prefill_gemm run M rows of N columns
+// on the skinny kernel.
+bool gemm_rows_skinny(int M, int N) { return skinny_rows(M, N); }
+
 // One skinny GEMM (M <= 16) over a weight block of three row segments
 // (ep.seg1, ep.seg2 bounds, scale0..2 their scales) with each segment's bf16
 // output in a buffer of its own: the batched decode step's q|k|v, whose
 // three row blocks the multi-row RoPE append reads. fp8: A is e4m3 codes with
 // the device scale a_scale (granite4_gemm_fp8's operands), else bf16
-// (granite4_prefill_gemm's). Not exported: layer_steps.hip calls it.
+// (granite4_prefill_gemm's). Not exported: layer_steps.hip calls it, where a
+// call per segment takes the skinny kernel too (gemm_rows_skinny), so that
+// each output is the same sum.
 int gemm_rows_split(bool fp8, const void* A, int lda, const float* a_scale, const uint8_t* W,
                     int M, int N, int K, const Granite4GemmEpilogue& ep, uint16_t* const out[3],
                     const int ld[3]) {
@@ -866,8 +872,6 @@ int gemm_rows_split(bool fp8, const void* A, int lda, const float* a_scale, cons
     a.seg_out[i] = out[i];
     a.seg_ld[i] = ld[i];
   }
-  // The skinny kernel whatever the width: each output is the same sum as in a
-  // call per segment, whose narrower outputs take it too.
   if (fp8) launch_skinny<true, kEpiBf16>(a, INT_MAX);
   else launch_skinny<false, kEpiBf16>(a, INT_MAX);
   return launch_status("gemm_rows_split");

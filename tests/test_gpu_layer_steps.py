@@ -353,6 +353,30 @@ def test_decode_step_multi_matches_one_by_one_and_oracle(ops):
     _close(host(log2), logits, "logits", fp8)
 
 
+@pytest.mark.parametrize("ops", ["bf16", "fp8"])
+def test_decode_step_multi_matches_one_by_one_past_4096_q_columns(ops):
+    """16 sessions of a model whose q has 5120 columns (40 query heads): past
+    4096 a q GEMM of its own takes a tile, and the step's q|k|v with it, so
+    that the step stays bit for bit the entry points one by one."""
+    fp8 = ops == "fp8"
+    note(f"decode step multi, 5120 q columns, ops={ops}")
+    n, stride = 16, 2048
+    m = Model(1024, 1024, 40, 10, 300, 2, 8, 128, stride, 16, 0x3A5 + fp8, max_pos=1024)
+    d_m, pos, pts, toks, keep = _multi_rows(m, n, 1024, 0x3A6)
+    start = m.arenas()
+    _multi_one_by_one(m, d_m, n, fp8)
+    hid1 = torch.empty((n, m.H), dtype=torch.bfloat16, device="cuda")
+    L.call("granite4_kernel_rmsnorm", m.steps.hidden, m.final_norm, m.eps, n, m.H, hid1)
+    want, want_arena = host(hid1).copy(), m.host_arenas()
+    m.restore(start)
+    hid2 = torch.empty_like(hid1)
+    m.steps.multi(d_m, n, L.OPS_FP8 if fp8 else L.OPS_BF16, hid2)
+    np.testing.assert_array_equal(host(hid2), want)
+    for a, b in zip(m.host_arenas(), want_arena):
+        for x, y in zip(a, b):
+            np.testing.assert_array_equal(x, y)
+
+
 def test_decode_step_multi_graph_replay_and_high_positions():
     """Config 2's position range: 8 sessions at positions in [0, 65536)
     (FP8 ops, int8 KV). Captured once, replayed at p and p + 1 (the
