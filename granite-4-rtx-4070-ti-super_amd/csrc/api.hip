@@ -72,7 +72,8 @@ int resident_blocks(const void* kernel, int threads) {
 
 namespace {
 // The current device's scratch pool (stream_scratch), made at its first use;
-// nullptr where it cannot be made.
+// nullptr where it cannot be made (the next call tries again: the device may
+// have been out of memory for a moment).
 hipMemPool_t scratch_pool() {
   static std::mutex mu;
   static std::map<int, hipMemPool_t> pools;
@@ -92,8 +93,8 @@ hipMemPool_t scratch_pool() {
     (void)hipMemPoolDestroy(pool);
     pool = nullptr;
   }
-  (void)hipGetLastError();
-  pools[dev] = pool;
+  if (pool != nullptr) pools[dev] = pool;
+  else (void)hipGetLastError();
   return pool;
 }
 }  // namespace

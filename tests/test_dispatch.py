@@ -25,3 +25,13 @@ def test_multi_step_qkv_takes_the_kernels_of_separate_calls(fp8):
         qkv = [k for k in map(kernel, step[:append]) if k[0].startswith("gemm_")]
         assert kv[0][0] == "gemm_skinny_kernel"  # k and v, or all three, in one launch
         assert qkv == (q if q == kv else q + kv), (hq, rows)
+
+
+# A key-split attention whose scratch pool cannot be made runs unsplit, and the
+# next call tries again; under capture it never splits.
+def test_prefill_attn_scratch_pool_failure_lasts_one_call():
+    step = ("prefill_attn", 17, 50000)
+    got = [names(s) for s in launched([("fail_pool_create", 1), step, step, ("capturing", 1), step,
+                                       ("capturing", 0), step])]
+    split = ["attn_prefill_kernel", "attn_prefill_combine_kernel"]
+    assert [[n for n, _ in s] for s in got if s] == [split[:1], split, split[:1], split]
