@@ -20,9 +20,9 @@
 //             max |act| for the per-tensor FP8 scale of the encode pass.
 //
 // Three kernels: up to 16 rows the skinny one (skinny_rows), from there on the
-// tile kernel (gemm_tile.h) where K is a multiple of its steps, and the two
-// general ones laid out next for other K (their times at layer shapes, below,
-// are from before the tile kernel took those).
+// tile kernel (gemm_tile.h) where K is a multiple of its steps and long enough
+// for its tiles, and the two general ones laid out next otherwise (their times
+// at layer shapes, below, are from before the tile kernel took those).
 //
 // Layout: 256-thread workgroups on 128 x 128 output tiles (swiglu: 64 act
 // columns = 64 gate + 64 up weight rows), 4 waves in 2 x 2, each wave 4 x 4
@@ -643,8 +643,6 @@ bool gemm_args_ok(const uint8_t* A, int lda, const uint8_t* W, int M, int N, int
 // sum's order differs from the large kernels' (K in NW parts); both are
 // held to the same parity bar.
 // ---------------------------------------------------------------------------
-constexpr int kSkinnyMaxM = 16;
-
 template <bool F8A, int EPI, int U, int NW>
 __global__ __launch_bounds__(NW * 64) void gemm_skinny_kernel(GemmArgs a) {
   __shared__ v4f s_acc[2][NW - 1][64];  // waves 1..NW-1's partial tiles (gate / up)
@@ -820,24 +818,49 @@ unsigned gemm_grid(long long tiles, int cap) {
   return static_cast<unsigned>(g > 0 ? g : 1);
 }
 
-// Whether M <= kSkinnyMaxM rows take the skinny kernel rather than a tile: it
+// Whether M <= kSkinnyMaxM rows take the skinny kernel rather than a tile. It
 // streams the weights best while its 16-column workgroups are at most one per
 // CU (K = 12800 down, 8 rows, us: skinny 12.5, tile 14.6; bf16 O 7.4 / 9.1), but
 // re-reads all activations in each, which past that costs more than the
-// tile's staging (FP8 / bf16 A q|k|v, 1.5 per CU: 2 rows 7.3 / 8.9 against 7.4 /
-// 9.7, 4 rows 8.3 / 9.9 against 7.3 / 9.7; 12800 columns, 3.1 per CU: 1 row
-// FP8 25.6 against 24.5, 16 rows bf16 25.6 against 14.2).
-bool skinny_rows(int M, int ncols) {
+// tile's staging, the sooner the more rows and K there are, and the later the
+// shorter the tile's K loop is (tile / skinny over 60 pairs of N and K from 4352
+// to 100352 columns, 1 to 16 rows):
+//   FP8, M K >= 16384: 0.63-1.05; M K = 4096: 1.00-1.28, 8192: 0.90-1.12. Past
+//   32768 columns 4 and 8 rows are 0.95-1.17, 12 and 16 0.79-1.00.
+//   bf16 up to two per CU, M K >= 16384: 0.65-1.01; M K = 8192: 0.95-1.13. Up to
+//   four, M K >= 768: 0.51-0.98. More: 4 rows and up 0.57-0.99, 2 rows 0.81-0.99 up
+//   to K = 4096 and 1.05-1.19 past it, 1 row 0.87-1.25.
+//   SwiGLU past two per CU, K >= 3584: 0.76-1.11; K = 2048: 1.00-1.28. Between one
+//   and a half and two 0.94-1.31. Up to one and a half, M K >= 256 for each
+//   workgroup past one per CU: 0.67-1.03.
+// Where only tiles of 128 rows and more fit (K not a multiple of 512, bf16 of
+// 256), the skinny kernel is up to 3 times as fast.
+enum class GemmKind { kFp8, kBf16, kSwiglu };
+bool skinny_rows(GemmKind kind, int M, int ncols, int K) {
   if (M > kSkinnyMaxM) return false;
   const int ntile = (ncols + 15) / 16;
-  return ntile <= kCUs || (ntile <= 2 * kCUs && M < 4);
+  if (ntile <= kCUs || K % (kind == GemmKind::kBf16 ? 256 : 512) != 0) return true;
+  const long long mk = static_cast<long long>(M) * K;
+  switch (kind) {
+    case GemmKind::kFp8: return mk < 16384 || M < (ntile > 8 * kCUs ? 12 : 4);
+    case GemmKind::kSwiglu:
+      if (ntile > 2 * kCUs) return K < 3584;
+      return 2 * ntile > 3 * kCUs || K < 1024 || mk < 256LL * (ntile - kCUs);
+    default:
+      if (K < 512) return true;
+      if (ntile <= 2 * kCUs) return mk < 16384 || M < 4;
+      if (ntile <= 4 * kCUs) return mk < 768;
+      return M < 2 || (M < 4 && K > 4096);
+  }
 }
 
 }  // namespace
 
 // Whether granite4_gemm_fp8 / granite4_prefill_gemm run M rows of N columns
 // on the skinny kernel.
-bool gemm_rows_skinny(int M, int N) { return skinny_rows(M, N); }
+bool gemm_rows_skinny(bool fp8, int M, int N, int K) {
+  return skinny_rows(fp8 ? GemmKind::kFp8 : GemmKind::kBf16, M, N, K);
+}
 
 // One skinny GEMM (M <= 16) over a weight block of three row segments
 // (ep.seg1, ep.seg2 bounds, scale0..2 their scales) with each segment's bf16
@@ -928,7 +951,7 @@ int granite4_gemm_fp8(int out, const uint8_t* A, int lda, const float* d_a_scale
     else if (deep == 3) go(gemm_fp8_kernel<E, 64, 3>, gemm_grid<E, 64, 3>(tiles, INT_MAX));
     else go(gemm_fp8_kernel<E, 64>, gemm_grid<E, 64>(tiles, INT_MAX));
   };
-  if (!skinny_rows(M, N) && launch_gemm_tile_fp8(out, a) != 0) return launch_status("granite4_gemm_fp8");
+  if (!skinny_rows(GemmKind::kFp8, M, N, K) && launch_gemm_tile_fp8(out, a) != 0) return launch_status("granite4_gemm_fp8");
   switch (out) {
     case GRANITE4_GEMM_BF16: run(std::integral_constant<int, kEpiBf16>{}); break;
     case GRANITE4_GEMM_F32: run(std::integral_constant<int, kEpiF32>{}); break;
@@ -979,7 +1002,7 @@ int granite4_prefill_gemm(int out, const uint16_t* A, int lda, const uint8_t* W,
     a.xcd_order = gemm_xcd_order(a.mt, gu);
     return gu;
   };
-  if (!skinny_rows(M, N) && launch_gemm_tile_bf16(out, a) != 0) return launch_status("granite4_prefill_gemm");
+  if (!skinny_rows(GemmKind::kBf16, M, N, K) && launch_gemm_tile_bf16(out, a) != 0) return launch_status("granite4_prefill_gemm");
   if (M <= kSkinnyMaxM) {
     if (out == GRANITE4_GEMM_BF16) launch_skinny<false, kEpiBf16>(a, INT_MAX);
     else if (out == GRANITE4_GEMM_F32) launch_skinny<false, kEpiF32>(a, INT_MAX);
@@ -1048,7 +1071,7 @@ int granite4_gemm_fp8_swiglu(const uint8_t* A, int lda, const float* d_a_scale,
   a.vec_out = true;
   a.partials = work_partials(d_work);
   const long long tiles = static_cast<long long>(a.mt) * a.nt;
-  unsigned grid = skinny_rows(M, I) ? 0 : launch_gemm_tile_fp8(kEpiSwiglu, a);
+  unsigned grid = skinny_rows(GemmKind::kSwiglu, M, I, K) ? 0 : launch_gemm_tile_fp8(kEpiSwiglu, a);
   if (grid == 0 && M <= kSkinnyMaxM) {
     grid = launch_skinny<true, kEpiSwiglu>(a, kMaxPartials);
   } else if (grid == 0) {

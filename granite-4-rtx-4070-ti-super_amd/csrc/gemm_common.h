@@ -89,11 +89,14 @@ __device__ __forceinline__ uint32_t pack_bf16_rne(float lo, float hi) { return p
 
 typedef __bf16 bf16x8_g __attribute__((ext_vector_type(8)));
 
+constexpr int kSkinnyMaxM = 16;  // rows of the skinny kernel at most
+
 // The LDS-staged tile kernels (gemm_tile.h): choose a tile for the shape and
 // launch it. epi: one of the kinds above (bf16 A: not kEpiSwiglu). Returns the
-// grid (swiglu: the number of partials written), or 0 where no tile takes the
-// arguments (K not a multiple of 256 FP8 / 128 bf16 elements, pitches beyond
-// 32-bit tile offsets); nothing is launched then.
+// grid (swiglu: the number of partials written), or 0, launching nothing, where
+// no tile takes the arguments (K not a multiple of 256 FP8 / 128 bf16 elements,
+// pitches beyond 32-bit tile offsets) or, above kSkinnyMaxM rows, the general
+// kernels are the faster ones (short K).
 unsigned launch_gemm_tile_fp8(int epi, const GemmArgs& a);
 unsigned launch_gemm_tile_bf16(int epi, const GemmArgs& a);
 

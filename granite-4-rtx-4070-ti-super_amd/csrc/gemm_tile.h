@@ -592,11 +592,30 @@ __global__ __launch_bounds__(256 * KS) __attribute__((amdgpu_waves_per_eu(KS, KS
 struct TileCost {
   float per_k, per_round, fixed;
 };
+// Where the configuration, the cheapest tile at a shape, is faster than the
+// general kernels (gemm.hip), measured over 19 K from 128 to 12800, 17 to 8192
+// rows and 256 to 25600 columns. Their prologue is shorter: a K of its own is
+// needed where their 128-row tiles are all on the chip at once (two per CU),
+// and where they take turns. Their rounds are of 512 tiles and not of 256: in
+// turns, `in_turn_us` (if set) is compared with theirs. (It is the time of the
+// same launch, fitted over K from 1024 on, and the choice between tiles stays
+// with `cost`, which is the closer one between them at layer shapes.)
+struct TileVsGeneral {
+  int at_once_k = 0, in_turn_k = 0;
+  TileCost in_turn_us = {};
+};
+
+// Tiles of the general kernels: 128 rows x 128 weight rows.
+inline long long general_tiles(const GemmArgs& a, bool glu) {
+  const long long n = glu ? (a.I + 63) / 64 : (a.N + 127) / 128;
+  return (a.M + 127) / 128 * n;
+}
 
 template <bool F8, int FM, int FN, int S, int KS, bool QUAD>
 struct TileConfig {
   using Shape = TileShape<F8, FM, FN, S, KS>;
   TileCost cost;
+  TileVsGeneral vs = {};
 
   static int cols(bool glu) { return (glu ? 16 : 32) * FN; }
   // Whether the kernel takes these arguments: whole pairs of steps for every
@@ -612,10 +631,24 @@ struct TileConfig {
     const int n = glu ? a.I : a.N;
     return static_cast<long long>((a.M + Shape::kBM - 1) / Shape::kBM) * ((n + cols(glu) - 1) / cols(glu));
   }
-  float predicted(const GemmArgs& a, bool glu) const {
+  static float time(const TileCost& c, const GemmArgs& a, bool glu) {
     const long long rounds = (tiles(a, glu) + kCUs - 1) / kCUs;
-    return static_cast<float>(rounds) * (cost.per_k * (static_cast<float>(a.K) / 4096.0f) + cost.per_round) +
-           cost.fixed;
+    return static_cast<float>(rounds) * (c.per_k * (static_cast<float>(a.K) / 4096.0f) + c.per_round) + c.fixed;
+  }
+  float predicted(const GemmArgs& a, bool glu) const { return time(cost, a, glu); }
+  // Whether the general kernels are the faster ones where this is the cheapest
+  // tile. general: their cost per round of 2 kCUs tiles.
+  bool loses(const GemmArgs& a, bool glu, const TileCost& general) const {
+    const long long g = general_tiles(a, glu), at_once = 2 * kCUs;
+    if (a.K < (g <= at_once ? vs.at_once_k : vs.in_turn_k)) return true;
+    // (SwiGLU 300 rows, I = 9600: 450 general tiles at once 16.2-42.1 us for K of
+    // 1536 to 4608, 450 128 x 128 tiles in two rounds 18.7-42.6)
+    if (g <= at_once) return glu && tiles(a, glu) > kCUs;
+    const long long rounds = (g + at_once - 1) / at_once;
+    return vs.in_turn_us.per_k > 0.0f &&
+           static_cast<float>(rounds) * (general.per_k * (static_cast<float>(a.K) / 4096.0f) + general.per_round) +
+                   general.fixed <
+               time(vs.in_turn_us, a, glu);
   }
   template <int EPI>
   static unsigned launch(GemmArgs a) {
@@ -632,9 +665,10 @@ struct TileConfig {
 };
 
 // Launches the configuration with the least predicted time of those that fit;
-// returns its grid, or 0 where none does (nothing is launched).
+// returns its grid, or 0 (nothing is launched) where none fits or, above
+// kSkinnyMaxM rows, the general kernels are the faster ones.
 template <int EPI, class... C>
-unsigned launch_cheapest(const GemmArgs& a, const C&... configs) {
+unsigned launch_cheapest(const GemmArgs& a, const TileCost& general, const C&... configs) {
   constexpr bool kGlu = EPI == kEpiSwiglu;
   float best = 0.0f;
   int pick = -1, i = 0;
@@ -649,7 +683,7 @@ unsigned launch_cheapest(const GemmArgs& a, const C&... configs) {
   unsigned grid = 0;
   i = 0;
   const auto go = [&](const auto& c) {
-    if (i++ == pick) grid = c.template launch<EPI>(a);
+    if (i++ == pick && (a.M <= kSkinnyMaxM || !c.loses(a, kGlu, general))) grid = c.template launch<EPI>(a);
   };
   (go(configs), ...);
   return grid;

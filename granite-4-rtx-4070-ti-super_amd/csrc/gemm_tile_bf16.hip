@@ -13,9 +13,13 @@ namespace {
 // rows 439 -> 285; O 64 rows 55.0 -> 10.4, 512 rows 55.2 -> 22.8, 8192 rows 308 ->
 // 208 (1.32 PFLOP/s; a library product of 8192^3 on the same card reaches
 // 1.28); down 64 rows 157 -> 22.3, 512 rows 158 -> 60.5, 8192 rows 901 -> 589.
-constexpr TileConfig<false, 8, 8, 2, 1, true> k256x256{{75.48f, 24.40f, -18.93f}};
-constexpr TileConfig<false, 8, 4, 3, 1, true> k256x128{{44.77f, 12.50f, -6.99f}};
-constexpr TileConfig<false, 4, 6, 4, 1, true> k128x192{{35.10f, 10.14f, -4.51f}};
+// Against the general kernel, at the cheapest tile's shapes, tile / general: 256 x
+// 256 in the mean 0.92 (up to 1.05) at K = 384, 0.98 (1.11) at 256; 256 x 128 at once
+// 1.00 at 512, 0.97 at 640, in turn 1.05 at 256, 0.98 at 384; 128 x 192 1.20 at 384,
+// 0.95 at 512; the smaller ones faster from where they fit (512).
+constexpr TileConfig<false, 8, 8, 2, 1, true> k256x256{{75.48f, 24.40f, -18.93f}, {384, 384}};
+constexpr TileConfig<false, 8, 4, 3, 1, true> k256x128{{44.77f, 12.50f, -6.99f}, {640, 384}};
+constexpr TileConfig<false, 4, 6, 4, 1, true> k128x192{{35.10f, 10.14f, -4.51f}, {512, 512}};
 constexpr TileConfig<false, 4, 4, 3, 2, true> k128x128{{22.34f, 11.67f, -7.56f}};
 constexpr TileConfig<false, 4, 3, 3, 2, false> k128x96{{19.94f, 7.63f, -2.81f}};
 constexpr TileConfig<false, 2, 4, 3, 2, true> k64x128{{15.63f, 7.11f, -4.25f}};
@@ -26,7 +30,11 @@ constexpr TileConfig<false, 1, 1, 4, 4, false> k32x32{{6.24f, 1.37f, 1.81f}};
 
 template <int EPI>
 unsigned go(const GemmArgs& a) {
-  return launch_cheapest<EPI>(a, k256x256, k256x128, k128x192, k128x128, k128x96, k64x128, k64x96, k64x64, k32x64,
+  // Tiles of fewer than 128 rows need a K that is a multiple of 256. Without
+  // them a small output leaves CUs idle, which a short K does not make up for
+  // (tile / general up to one general tile per CU: 1.07 at K = 640, 0.98 at 896).
+  if (a.M > kSkinnyMaxM && a.K % 256 != 0 && a.K < 896 && general_tiles(a, false) <= kCUs) return 0;
+  return launch_cheapest<EPI>(a, TileCost{}, k256x256, k256x128, k128x192, k128x128, k128x96, k64x128, k64x96, k64x64, k32x64,
                               k32x32);
 }
 

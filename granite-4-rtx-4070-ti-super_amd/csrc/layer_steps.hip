@@ -41,7 +41,7 @@
 
 namespace g4 {
 // gemm.hip: whether a GEMM of these rows and columns takes the skinny kernel.
-bool gemm_rows_skinny(int M, int N);
+bool gemm_rows_skinny(bool fp8, int M, int N, int K);
 // gemm.hip: the skinny GEMM (rows <= 16) with a bf16 output per row segment.
 int gemm_rows_split(bool fp8, const void* A, int lda, const float* a_scale, const uint8_t* W,
                     int M, int N, int K, const Granite4GemmEpilogue& ep, uint16_t* const out[3],
@@ -144,20 +144,20 @@ int qkv_gemm(const Granite4DecodeModel* m, const Granite4DecodeLayer& y,
     return gemm(y.wq, nq + 2 * nk, e);
   }
   // Rows of a weight block into buffers of their own: one launch, the same sums
-  // as a call per matrix where those take the skinny kernel too. They do not
-  // past 4096 columns at 4 rows and more: a model with that many q columns
-  // (more than 32 heads) takes a tile for q, and the one launch for k and v (40
+  // as a call per matrix where those take the skinny kernel too. Past 4096
+  // columns they may not: a model with that many q columns (more than 32
+  // heads) takes a tile for q, and the one launch for k and v (H 4096, 40
   // heads, per layer at short contexts, us: 4 rows 63 -> 67 FP8, 69 bf16; 16
   // rows 74 -> 77, 77 -> 82; 32 heads unchanged).
   const bool contiguous_w = y.wk == y.wq + static_cast<size_t>(nq) * H &&
                             y.wv == y.wk + static_cast<size_t>(nk) * H;
-  const bool split = contiguous_w && rows <= kSkinnyRows && g4::gemm_rows_skinny(rows, nk);
+  const bool split = contiguous_w && rows <= kSkinnyRows && g4::gemm_rows_skinny(fp8, rows, nk, H);
   const auto rows_split = [&](const uint8_t* W, int N, const Granite4GemmEpilogue& e, uint16_t* const outs[3],
                               const int lds[3]) {
     return fp8 ? g4::gemm_rows_split(true, b->codes, H, b->scales, W, rows, N, H, e, outs, lds)
                : g4::gemm_rows_split(false, b->normed, H, nullptr, W, rows, N, H, e, outs, lds);
   };
-  if (split && g4::gemm_rows_skinny(rows, nq)) {
+  if (split && g4::gemm_rows_skinny(fp8, rows, nq, H)) {
     const Granite4GemmEpilogue e = epi_bf16(y.sq, y.sk, y.sv, nq, nq + nk, q_out, ldq);
     uint16_t* const outs[3] = {q_out, k_out, v_out};
     const int lds[3] = {ldq, ldk, ldv};

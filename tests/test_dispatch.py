@@ -35,3 +35,41 @@ def test_prefill_attn_scratch_pool_failure_lasts_one_call():
                                        ("capturing", 0), step])]
     split = ["attn_prefill_kernel", "attn_prefill_combine_kernel"]
     assert [[n for n, _ in s] for s in got if s] == [split[:1], split, split[:1], split]
+
+
+# Where the tile kernel is the slower one (a K too short for its pipeline, or a
+# last round of tiles nearly empty; by the factor given), the call takes the
+# kernel that is faster; layer shapes keep the tile.
+FASTER = [  # FP8 (None: SwiGLU), rows, columns, K, kernel
+    (True, 128, 1024, 256, "gemm_fp8_kernel"),      # 2.4
+    (True, 700, 4096, 512, "gemm_fp8_kernel"),      # 1.5
+    (True, 1000, 2560, 1024, "gemm_fp8_kernel"),    # 1.3
+    (True, 96, 7168, 1280, "gemm_fp8_kernel"),      # 1.1
+    (True, 32, 25600, 2048, "gemm_fp8_kernel"),     # 1.15
+    (True, 300, 4096, 1792, "gemm_fp8_kernel"),     # 1.07
+    (True, 4, 8192, 1280, "gemm_skinny_kernel"),    # 1.7
+    (True, 16, 8192, 512, "gemm_skinny_kernel"),    # 2.1
+    (True, 1, 25600, 2048, "gemm_skinny_kernel"),   # 1.2
+    (False, 128, 1024, 128, "gemm_bf16w_kernel"),   # 2.1
+    (False, 700, 2560, 256, "gemm_bf16w_kernel"),   # 1.4
+    (False, 300, 1024, 640, "gemm_bf16w_kernel"),   # 1.1
+    (False, 4, 8192, 1152, "gemm_skinny_kernel"),   # 2.9
+    (False, 8, 6144, 512, "gemm_skinny_kernel"),    # 1.2
+    (None, 300, 2048, 256, "gemm_fp8_kernel"),      # 2.1
+    (None, 300, 8192, 2560, "gemm_fp8_kernel"),     # 1.1
+    (None, 300, 9600, 2560, "gemm_fp8_kernel"),     # 1.1
+    (None, 8, 8192, 4096, "gemm_skinny_kernel"),    # 1.2
+    (True, 2561, 6144, 4096, "gemm_fp8_kernel"),    # 1.3
+    (None, 832, 12800, 4096, "gemm_fp8_kernel"),    # 1.08
+    (True, 512, 4096, 12800, "gemm_tile_kernel"), (True, 8192, 6144, 4096, "gemm_tile_kernel"),
+    (True, 16, 6144, 4096, "gemm_tile_kernel"), (False, 1000, 6144, 4096, "gemm_tile_kernel"),
+    (False, 17, 4096, 4096, "gemm_tile_kernel"), (False, 16, 100352, 4096, "gemm_tile_kernel"),
+    (None, 8192, 12800, 4096, "gemm_tile_kernel"), (None, 1, 12800, 4096, "gemm_tile_kernel"),
+    (True, 8, 4096, 12800, "gemm_skinny_kernel"), (False, 16, 4096, 4096, "gemm_skinny_kernel"),
+]
+
+
+def test_gemm_takes_the_faster_kernel():
+    got = launched([("gemm_swiglu", m, n, k) if fp8 is None else ("gemm", fp8, m, n, k)
+                    for fp8, m, n, k, _ in FASTER])
+    assert [(*f[:4], names(s)[0][0]) for f, s in zip(FASTER, got)] == FASTER
