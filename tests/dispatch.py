@@ -58,9 +58,9 @@ class Steps:
     def gemm_swiglu(self, m, i, k):
         self.L.call("granite4_gemm_fp8_swiglu", ADDR, k, ADDR, ADDR, m, i, k, 1.0, 1.0, ADDR, None, None, ADDR)
 
-    def prefill_attn(self, rows, base, bits=8, hk=8):
+    def prefill_attn(self, rows, base, window=0, hk=8, bits=8):
         self.L.call("granite4_prefill_attn", ADDR, rows, 4 * hk, hk, 128, 1 / 128, ADDR, ADDR, ADDR, ADDR, bits,
-                    128, 1 << 16, base, ADDR, 0, ADDR)
+                    128, 1 << 16, base, ADDR, window, ADDR)
 
     def multi_step(self, hidden, inter, hq, hk, rows, fp8):
         """granite4_decode_step_multi of one layer, q|k|v one block."""

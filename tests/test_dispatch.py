@@ -73,3 +73,22 @@ def test_gemm_takes_the_faster_kernel():
     got = launched([("gemm_swiglu", m, n, k) if fp8 is None else ("gemm", fp8, m, n, k)
                     for fp8, m, n, k, _ in FASTER])
     assert [(*f[:4], names(s)[0][0]) for f, s in zip(FASTER, got)] == FASTER
+
+
+def prefill_plan(step):
+    """(positions per workgroup, key splits) of a prefill attention's launches."""
+    _, (_, _, blocks, _, ksp) = kernel(step[0][0])
+    assert len(step) == (1 if step[0][1][2] == 1 else 2)
+    return 16 if ksp == 2 else 32 * blocks, step[0][1][2]
+
+
+# Behind a window most workgroups are as long as the longest: their mean length
+# is not half of it (us with the plan of a chunk that grows throughout / this one).
+@pytest.mark.parametrize("rows,base,window,hk,plan", [
+    (1300, 0, 1024, 8, (32, 1)),    # 50.0 / 42.1
+    (2000, 0, 1024, 8, (64, 1)),    # 69.6 / 57.9
+    (900, 0, 256, 8, (32, 1)),      # 24.1 / 17.2 (split before)
+    (4096, 0, 1024, 2, (32, 1)),    # 52.3 / 38.4
+    (2000, 0, 0, 8, (32, 1)), (2000, 0, 4096, 8, (32, 1))])
+def test_prefill_plan_behind_a_window(rows, base, window, hk, plan):
+    assert prefill_plan(launched([("prefill_attn", rows, base, window, hk)])[0]) == plan
