@@ -1785,17 +1785,26 @@ size_t prefill_split_bytes(int rows, int Hq, int nsp) {
 // A short chunk at the end of a long context (a conversation's next turn) has
 // few workgroups, each walking the whole context: 17 rows at 50000 took 1.17
 // ms on 16 CUs. There the keys are split over workgroups too, and a second
-// launch combines the partials. A split holds at least 4 tiles.
+// launch combines the partials. The longest workgroup's splits hold at least 4
+// tiles in the mean; the causal rows before it split their fewer tiles as many
+// ways, and some of their splits are empty.
 //
 // The plan is the one with the least predicted time: a tile's time in each form
 // (measured, us: 64 positions 2.95, or 2.45 where a CU runs several workgroups
 // in turn, 32 positions 2.1, 16 positions 2.9 per two tiles) times the tiles
 // that the busiest CU runs: the longest workgroup's, or the mean load, or full
-// rounds of the shortest ones (longest first, the CUs even out). Splits add a launch, and each partial
-// written and read at 4 TB/s. Within 9 % of the best of the three forms and up
-// to 16 splits at 20 shapes of 17 to 4096 rows. Against 64 positions wherever
-// those give every CU a workgroup, else 32, else 16 (int8 from 0, us): 1000
-// rows 37.9 -> 31.3, 2000 rows 101.5 -> 76.7, 2500 rows 124 -> 114.
+// rounds of the shortest ones (longest first, the CUs even out). Within 9 % of
+// the best of the three forms at 20 shapes of 17 to 4096 rows. Against 64
+// positions wherever those give every CU a workgroup, else 32, else 16 (int8
+// from 0, us): 1000 rows 37.9 -> 31.3, 2000 rows 101.5 -> 76.7, 2500 rows 124 -> 114.
+//
+// Splits add a launch, 6 us, and each partial written and read at 4 TB/s, which
+// finds their number. Against the whole form they count with 8 us and 3.6 TB/s,
+// and with 20 us at least, which the host needs for such a call (the scratch,
+// two launches) however short its kernels are. Without that 108 of 1596 shapes
+// were split that ran more than 5 % faster whole, some slower than with no splits
+// at all (1 row after 700 positions 26 to 33 us for 19.5, 900 rows after 1000 72
+// for 60.5); with it 49.
 PrefillPlan prefill_plan(int rows, int base, int window, int Hk, bool may_split) {
   constexpr int kPositions[] = {64, 32, 16};
   constexpr double kPerTile[] = {2.95, 2.1, 1.45}, kPerTileInTurn[] = {2.45, 2.1, 1.45};
@@ -1803,8 +1812,9 @@ PrefillPlan prefill_plan(int rows, int base, int window, int Hk, bool may_split)
     const int span = window > 0 && window < end - pos ? window + pos : end;
     return (span + kTile - 1) / kTile;
   };
-  PrefillPlan p{PrefillPlan::k64, 1};
-  double best = 0.0;
+  constexpr double kSplitHostUs = 20.0;
+  PrefillPlan plan[2] = {{PrefillPlan::k64, 1}, {PrefillPlan::k64, 1}};  // whole, split
+  double best[2] = {0.0, 0.0}, split = 0.0;
   for (const auto form : {PrefillPlan::k64, PrefillPlan::k32, PrefillPlan::k16x2}) {
     const int pos = kPositions[form];
     const long long blocks = static_cast<long long>((rows + pos - 1) / pos) * Hk;
@@ -1815,20 +1825,26 @@ PrefillPlan prefill_plan(int rows, int base, int window, int Hk, bool may_split)
     const double growing = window > 0 && window < base + rows ? std::max(window - base, 0) / static_cast<double>(rows) : 1.0;
     const double mean_tiles = longest - 0.5 * growing * (longest - shortest);
     for (int nsp = 1; nsp == 1 || (nsp <= kPrefillMaxSplits && nsp * 4 <= longest); ++nsp) {
-      double extra = 0.0;
+      double extra = 0.0, against = 0.0;  // of the splits; against the whole form more
       if (nsp > 1) {
         const double bytes = static_cast<double>(prefill_split_bytes(rows, 4 * Hk, nsp));
         if (!may_split || form == PrefillPlan::k32 || bytes > static_cast<double>(kPrefillSplitBytes)) break;
         extra = 6.0 + 2.0 * bytes / 4e6;
+        against = 2.0 + 2.0 * bytes * (1.0 / 3.6e6 - 1.0 / 4e6);
       }
       const double wgs = static_cast<double>(blocks) * nsp, top = std::ceil(static_cast<double>(longest) / nsp);
       const double mean = wgs / kCUs * mean_tiles / nsp;
       const double rounds = std::ceil(wgs / kCUs) * std::ceil(static_cast<double>(shortest) / nsp);
       const double t = std::max(kPerTile[form] * top, kPerTileInTurn[form] * std::max(mean, rounds)) + extra;
-      if (best == 0.0 || t < 0.95 * best) best = t, p = PrefillPlan{form, nsp};
+      const int s = nsp > 1;
+      if (best[s] == 0.0 || t < 0.95 * best[s]) {
+        best[s] = t;
+        plan[s] = PrefillPlan{form, nsp};
+        if (s == 1) split = std::max(t + against, kSplitHostUs);
+      }
     }
   }
-  return p;
+  return plan[best[1] > 0.0 && split < best[0]];
 }
 
 template <int BITS>

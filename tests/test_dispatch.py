@@ -92,3 +92,17 @@ def prefill_plan(step):
     (2000, 0, 0, 8, (32, 1)), (2000, 0, 4096, 8, (32, 1))])
 def test_prefill_plan_behind_a_window(rows, base, window, hk, plan):
     assert prefill_plan(launched([("prefill_attn", rows, base, window, hk)])[0]) == plan
+
+
+# Key splits only where the call gains by them: its scratch and its two launches
+# take the host 20 us, and the partials their share of the memory's time (us
+# split / whole).
+@pytest.mark.parametrize("rows,base,hk,plan", [
+    (1, 700, 8, (16, 1)),       # 33.1 / 19.5
+    (64, 700, 8, (16, 1)),      # 26.8 / 20.3
+    (128, 500, 1, (16, 1)),     # 25.3 / 17.7
+    (1000, 1000, 8, (32, 1)),   # 79.2 / 63
+    (2000, 500, 4, (16, 1)),    # 84.5 / 71.9
+    (8, 3000, 8, (16, 10)), (17, 50000, 8, (64, 61)), (500, 20000, 8, (64, 4))])
+def test_prefill_plan_splits_keys_where_they_gain(rows, base, hk, plan):
+    assert prefill_plan(launched([("prefill_attn", rows, base, 0, hk)])[0]) == plan

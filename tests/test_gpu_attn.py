@@ -624,6 +624,22 @@ def test_prefill_attn_key_splits(rows, bits, group, window):
         check(host(args[6]).view(np.uint16), want, vmax(cv, vs, bits), f"captured rows {rows}")
 
 
+# 17 rows after 50000 positions: 61 key splits, so that the combine reads past its
+# first chunks of eight partials, the last of them part full.
+@pytest.mark.parametrize("bits,group", [(8, 128), (16, 128)])
+def test_prefill_attn_61_key_splits(bits, group):
+    note(f"prefill attn 61 key splits bits={bits}")
+    rows, base = 17, 50000
+    pages = (base + rows + 15) // 16
+    stride = 16 * pages
+    ck, cv, ks, vs = make_cache(bits, group, stride, 0xA6 + bits)
+    pt = ol.row_table(np.random.default_rng(bits).permutation(pages).astype(np.int32), stride)
+    q = ol.normal_bf16(0xA7, 0.0, 1.0, rows * HQ * D).reshape(rows, HQ * D)
+    want = ol.prefill_attn(q, ck, cv, ks, vs, bits, group, stride, base, pt=pt, scale=1.0 / 16, Hk=HK)
+    got = run_prefill(q, ck, cv, ks, vs, bits, group, stride, base, d_pt=dev(pt))
+    check(got, want, vmax(cv, vs, bits), "61 key splits")
+
+
 # Chunks from position 0, whose workgroups differ most in length: 1000 rows run
 # the 16-position form over two rounds of workgroups, 2000 rows the 32-position
 # one; one KV head leaves CUs for key splits, of which the first rows' shares
