@@ -1,6 +1,7 @@
 """Which kernels the entry points launch, without a GPU (dispatch.py)."""
 import pytest
 
+import gemm_tile_shapes as shapes
 from dispatch import kernel, launched
 
 
@@ -106,3 +107,32 @@ def test_prefill_plan_behind_a_window(rows, base, window, hk, plan):
     (8, 3000, 8, (16, 10)), (17, 50000, 8, (64, 61)), (500, 20000, 8, (64, 4))])
 def test_prefill_plan_splits_keys_where_they_gain(rows, base, hk, plan):
     assert prefill_plan(launched([("prefill_attn", rows, base, 0, hk)])[0]) == plan
+
+
+# The shapes of the tile GEMM's test run the configurations that they name, as
+# many tiles per workgroup as they say; the K padded copies that they are
+# compared with, and the short K, run the other kernels.
+def test_gemm_tile_shapes_run_the_named_tiles():
+    todo = ([(True, *s) for s in shapes.FP8] + [(False, *s) for s in shapes.BF16] +
+            [(None, *s) for s in shapes.SWIGLU])
+
+    def step(fp8, m, n, k):
+        return ("gemm_swiglu", m, n, k) if fp8 is None else ("gemm", fp8, m, n, k)
+
+    for (fp8, m, n, k, fragments, turns), got in zip(todo, launched([step(*t[:4]) for t in todo])):
+        (name, args), grid = kernel(got[0][0]), got[0][1][0]
+        assert (name, tuple(args[2:4])) == ("gemm_tile_kernel", fragments), (fp8, m, n, k)
+        count = shapes.tiles(m, n, fragments, fp8 is None)
+        assert grid == min(count, 256) and -(-count // grid) == turns, (fp8, m, n, k, count)
+    other = [step(t[0], t[1], t[2], t[3] + (32 if t[0] is False else 128)) for t in todo]
+    other += [step(f, *s) for f, l in ((True, shapes.FP8_OTHER), (False, shapes.BF16_OTHER),
+                                       (None, shapes.SWIGLU_OTHER)) for s in l]
+    for s, got in zip(other, launched(other)):
+        assert kernel(got[0][0])[0] != "gemm_tile_kernel", s
+
+
+# The bf16 general kernel's two residual forms: loaded at a tile's start, or
+# after its K loop where tiles outnumber the resident workgroups.
+def test_prefill_gemm_residual_forms():
+    got = launched([("gemm", False, 200, 256, 480, 2), ("gemm", False, 2100, 4096, 128, 2)])
+    assert [names(s) for s in got] == [[("gemm_bf16w_kernel", [2, 0])], [("gemm_bf16w_kernel", [2, 1])]]

@@ -90,13 +90,15 @@ def run_gemm(kind, A, a_scale, W, scales=(1.0, 1.0, 1.0), segs=None, residual=No
     return host(out)
 
 
-# Fewer than 256 output tiles of 128 x 128 take the 128 x 64 tile form, and
-# where those give each CU at most one tile, K split between the two halves of
-# a 512-thread workgroup (K = 128 and 384: an odd count of 128-wide K tiles,
-# half 1 idle in the last step); the 1100-row shape (9 x 32 = 288 tiles) the
-# 128 x 128 form.
+# The general kernel where K is too short for a tile or no multiple of its
+# steps: fewer than 256 output tiles of 128 x 128 take its 128 x 64 tile form,
+# and where those give each CU at most one tile, K split between the two halves
+# of a 512-thread workgroup (K = 384: an odd count of 128-wide K tiles, half 1
+# idle in the last step); the 1100-row shape (9 x 32 = 288 tiles) the 128 x 128
+# form. (300, 520, 1024) and (257, 1024, 4096) take a 64 x 32 tile of the tile
+# kernel.
 # M <= 16 takes the skinny kernel (16-column workgroups, K in quarters: 384 gives
-# quarters of 0, 1, 1 and 1 steps), M = 17 the tiled one.
+# quarters of 0, 1, 1 and 1 steps), M = 17 the general one.
 SHAPES = [(1, 128, 128), (70, 136, 256), (128, 256, 512), (300, 520, 1024), (257, 1024, 4096),
           (1100, 4096, 128), (96, 192, 384), (8, 136, 4096), (16, 520, 384), (17, 520, 384),
           (5, 4096, 12800)]

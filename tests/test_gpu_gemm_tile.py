@@ -1,18 +1,21 @@
 """The tile GEMM (granite4_gemm_fp8, granite4_gemm_fp8_swiglu and
-granite4_prefill_gemm from 17 rows on) at the edges of its tiles and rings.
+granite4_prefill_gemm, most calls of 17 rows and more) at the edges of its tiles
+and rings.
 
 Operands are small multiples of 1/2, so every partial sum is a multiple of 1/4
 below 2^24 / 4 and exact in f32 in any order: outputs are compared with a
 float64 product bit for bit, and with the general kernels bit for bit, which
 the same product reaches with zero columns appended to K (to an odd count of
-128 for FP8, to no multiple of 64 for bf16). Each shape names the tile that its
-predicted cost selects.
+128 for FP8, to no multiple of 64 for bf16). The shapes (gemm_tile_shapes.py)
+name the tile that each runs, and several have more tiles than workgroups: the
+ring then runs on from a tile into the next one, or is filled again (K groups).
 """
 import sys
 
 import pytest
 import torch
 
+import gemm_tile_shapes as shapes
 from pkg import layerops
 
 pytestmark = pytest.mark.gpu
@@ -48,36 +51,8 @@ def pitched(M, N, gap, dtype, fill):
     return whole[:, :N], whole
 
 
-FP8_SHAPES = [
-    (17, 40, 256),       # 256 x 256, fewer steps than two rounds of its ring
-    (17, 136, 512),      # 128 x 192
-    (2049, 2600, 256),   # 256 x 256, one row in the last tile row
-    (700, 8200, 512),    # 256 x 128, 8 columns in the last tile column
-    (129, 12808, 1536),  # 128 x 128
-    (65, 12808, 1024),   # 128 x 64, two K groups
-    (129, 8200, 1024),   # 64 x 128
-    (65, 8200, 1024),    # 64 x 96
-    (65, 4104, 1024),    # 64 x 64
-    (33, 40, 1536),      # 64 x 32
-    (16, 12808, 512),    # 16 rows, more skinny workgroups than CUs
-]
-BF16_SHAPES = [
-    (17, 38, 128),       # 256 x 256; odd groups of 8 columns, even pitch
-    (129, 136, 256),     # 128 x 192
-    (700, 8200, 256),    # 256 x 128
-    (129, 12806, 512),   # 128 x 128
-    (65, 8198, 512),     # 64 x 128
-    (33, 136, 512),      # 64 x 64
-    (33, 42, 1024),      # 32 x 64
-    (17, 40, 2048),      # 32 x 32, four K groups
-    (193, 4104, 2048),   # 64 x 96
-    (700, 3080, 2048),   # 128 x 96
-    (2500, 2600, 128),   # 256 x 256, several tiles per workgroup
-    (9, 8200, 512),      # 9 rows, more skinny workgroups than CUs
-]
-
-
-@pytest.mark.parametrize("fp8,M,N,K", [(True, *s) for s in FP8_SHAPES] + [(False, *s) for s in BF16_SHAPES])
+@pytest.mark.parametrize("fp8,M,N,K", [(True, *s[:3]) for s in shapes.FP8 + shapes.FP8_OTHER] +
+                         [(False, *s[:3]) for s in shapes.BF16 + shapes.BF16_OTHER])
 def test_gemm_tile_equals_general_path(fp8, M, N, K):
     print(f"gemm tile {'fp8' if fp8 else 'bf16'} M={M} N={N} K={K}", flush=True)
     pad = 128 if fp8 else 32
@@ -119,9 +94,7 @@ def test_gemm_tile_equals_general_path(fp8, M, N, K):
             assert torch.equal(got[0], got[1]), (kind, gap)
 
 
-# 16 FN gate and up columns per tile: 256 x 256 tiles hold 128 of I, 64 x 64 ones 32.
-@pytest.mark.parametrize("M,I,K", [(17, 40, 256), (17, 136, 512), (129, 8200, 512), (65, 4104, 1024),
-                                   (300, 520, 1536), (2049, 1288, 256), (16, 8200, 512)])
+@pytest.mark.parametrize("M,I,K", [s[:3] for s in shapes.SWIGLU + shapes.SWIGLU_OTHER])
 def test_gemm_tile_swiglu_equals_general_path(M, I, K):
     print(f"gemm tile swiglu M={M} I={I} K={K}", flush=True)
     A, W, a, w = operands(M, 2 * I, K, 128, True)

@@ -103,10 +103,11 @@ def test_prefill_gemm_f32_out(M, N, K):
     assert np.all(err <= bound(A, W, sc, None) + np.abs(y) * 2.0 ** -23)
 
 
-# 200 x 256: 4 tiles, the residual prefetched at each tile's start; 2100 x
-# 4096: 544 tiles, more than the 512 workgroups resident at two per CU, so the
-# form that loads the residual after the K loop runs.
-@pytest.mark.parametrize("M,N,K", [(200, 256, 512), (2100, 4096, 128), (8, 4096, 4096)])
+# 200 x 256: 64 x 64 tiles of the tile kernel at K = 512, and at 480 4 tiles of the
+# general one, the residual prefetched at each tile's start; 2100 x 4096: 544
+# tiles, more than the 512 workgroups resident at two per CU, so the form that
+# loads the residual after the K loop runs.
+@pytest.mark.parametrize("M,N,K", [(200, 256, 512), (200, 256, 480), (2100, 4096, 128), (8, 4096, 4096)])
 def test_prefill_gemm_residual_in_place(M, N, K):
     """kResidual, the O / down projection: hidden = bf16(hidden + rs * y), in place."""
     note(f"prefill_gemm residual M={M} N={N} K={K}")
