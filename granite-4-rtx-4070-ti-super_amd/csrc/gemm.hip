@@ -825,8 +825,10 @@ unsigned gemm_grid(long long tiles, int cap) {
 // tile's staging, the sooner the more rows and K there are, and the later the
 // shorter the tile's K loop is (tile / skinny over 60 pairs of N and K from 4352
 // to 100352 columns, 1 to 16 rows):
-//   FP8, M K >= 16384: 0.63-1.05; M K = 4096: 1.00-1.28, 8192: 0.90-1.12. Past
-//   32768 columns 4 and 8 rows are 0.95-1.17, 12 and 16 0.79-1.00.
+//   FP8 up to two per CU, M K >= 32768: 0.69-1.03; M K = 16384: 0.94-1.05, and
+//   1.12 where the weights come from memory (q|k|v 4 rows 9.6 / 10.7 us). More,
+//   M K >= 16384: 0.63-1.03; 4096: 1.00-1.28, 8192: 0.90-1.12. Past 32768 columns 4
+//   and 8 rows are 0.95-1.17, 12 and 16 0.79-1.00.
 //   bf16 up to two per CU, M K >= 16384: 0.65-1.01; M K = 8192: 0.95-1.13. Up to
 //   four, M K >= 768: 0.51-0.98. More: 4 rows and up 0.57-0.99, 2 rows 0.81-0.99 up
 //   to K = 4096 and 1.05-1.19 past it, 1 row 0.87-1.25.
@@ -842,7 +844,7 @@ bool skinny_rows(GemmKind kind, int M, int ncols, int K) {
   if (ntile <= kCUs || K % (kind == GemmKind::kBf16 ? 256 : 512) != 0) return true;
   const long long mk = static_cast<long long>(M) * K;
   switch (kind) {
-    case GemmKind::kFp8: return mk < 16384 || M < (ntile > 8 * kCUs ? 12 : 4);
+    case GemmKind::kFp8: return mk < (ntile > 2 * kCUs ? 16384 : 32768) || M < (ntile > 8 * kCUs ? 12 : 4);
     case GemmKind::kSwiglu:
       if (ntile > 2 * kCUs) return K < 3584;
       return 2 * ntile > 3 * kCUs || K < 1024 || mk < 256LL * (ntile - kCUs);

@@ -24,7 +24,7 @@ FP8 = [
     (17, 8200, 1024, (2, 2), 1),
     (33, 40, 1536, (2, 1), 1),
     (17, 8, 1024, (2, 1), 1),
-    (16, 6152, 1024, (2, 1), 1),      # 16 rows, more skinny workgroups than CUs
+    (16, 6152, 2048, (2, 1), 1),      # 16 rows, more skinny workgroups than CUs
 ]
 BF16 = [
     (257, 16392, 512, (8, 8), 1),

@@ -51,6 +51,7 @@ FASTER = [  # FP8 (None: SwiGLU), rows, columns, K, kernel
     (True, 4, 8192, 1280, "gemm_skinny_kernel"),    # 1.7
     (True, 16, 8192, 512, "gemm_skinny_kernel"),    # 2.1
     (True, 1, 25600, 2048, "gemm_skinny_kernel"),   # 1.2
+    (True, 4, 6144, 4096, "gemm_skinny_kernel"),    # 1.1 (weights from memory)
     (False, 128, 1024, 128, "gemm_bf16w_kernel"),   # 2.1
     (False, 700, 2560, 256, "gemm_bf16w_kernel"),   # 1.4
     (False, 300, 1024, 640, "gemm_bf16w_kernel"),   # 1.1

@@ -361,7 +361,7 @@ def test_decode_step_multi_matches_one_by_one_past_4096_q_columns(ops):
     fp8 = ops == "fp8"
     note(f"decode step multi, 5120 q columns, ops={ops}")
     n, stride = 16, 2048
-    m = Model(1024, 1024, 40, 10, 300, 2, 8, 128, stride, 16, 0x3A5 + fp8, max_pos=1024)
+    m = Model(2048, 1024, 40, 10, 300, 2, 8, 128, stride, 16, 0x3A5 + fp8, max_pos=1024)
     d_m, pos, pts, toks, keep = _multi_rows(m, n, 1024, 0x3A6)
     start = m.arenas()
     _multi_one_by_one(m, d_m, n, fp8)
