@@ -1081,11 +1081,10 @@ __global__ __launch_bounds__(kCombineThreads) void attn_combine_kernel(AttnArgs 
 // output is bf16(o * (1 / l)) (prefill_gemm.cu:930-940).
 // ---------------------------------------------------------------------------
 constexpr int kKPitch = kHd + 8;  // K tile pitch (bf16): 272 B, 16 rows on distinct banks
-// Waves per prefill workgroup (template parameter W): 8. Staging a tile's K / V into LDS is
-// split over all of them, so more waves sharing a tile cost less staging per
-// score; fewer waves per workgroup give short prompts more workgroups.
-// Measured: T=8192 at 57344 K5V4 8 waves 23.6 ms, 4 waves 48.5 ms; T=512
-// int8 (128 8-wave workgroups) 23.3 us, 4 waves 21.5 us.
+// Every prefill workgroup has 8 waves (template parameter W): staging a tile's K /
+// V into LDS is split over all of them (with the first form of this kernel
+// T=8192 at 57344 K5V4 took 23.6 ms with 8 waves, 48.5 with 4). Short prompts get
+// more workgroups from the form whose two 4-wave groups share the keys.
 
 struct PrefillArgs {
   const uint16_t* q;  // [rows][Hq][128]

@@ -519,8 +519,7 @@ __global__ __launch_bounds__(256 * KS) __attribute__((amdgpu_waves_per_eu(KS, KS
 #pragma unroll
         for (int c = 0; c < kCols / 16; ++c) column_block(c, std::false_type{});
       }
-      if (EPI == kEpiResidual && KS > 1 && b >= KS) load_res(b);
-      if (EPI == kEpiResidual && KS > 1 && b > 0 && b < KS) load_res(b);
+      if (EPI == kEpiResidual && KS > 1 && b > 0) load_res(b);
       if (EPI == kEpiResidual && KS == 1 && b + 1 < FM) load_res(b + 1);
       tile_reads_wait();
 #pragma unroll

@@ -7,12 +7,13 @@ namespace {
 
 // Rows x weight rows of a tile, and the costs fitted to 76 shapes (N x K of
 // q|k|v 6144 x 4096, O 4096 x 4096, down 4096 x 12800, one of gate|up 12800 x
-// 4096, 17 to 8192 rows, us; the choice by them is within 8 %, in the mean 0.3 %,
-// of the best of these). Measured against the 128 x 128 kernel of gemm.hip, us:
-// q|k|v 64 rows 52.4 -> 11.3, 512 rows 53.6 -> 28.2, 1000 rows 66.9 -> 47.0, 8192
-// rows 439 -> 285; O 64 rows 55.0 -> 10.4, 512 rows 55.2 -> 22.8, 8192 rows 308 ->
-// 208 (1.32 PFLOP/s; a library product of 8192^3 on the same card reaches
-// 1.28); down 64 rows 157 -> 22.3, 512 rows 158 -> 60.5, 8192 rows 901 -> 589.
+// 4096, 17 to 8192 rows, us, the weights in the cache; the choice by them is
+// within 8 %, in the mean 0.3 %, of the best of these). Measured against the 128 x
+// 128 kernel of gemm.hip, us, the operands rotated through 700 MB: q|k|v 64 rows
+// 54.4 -> 15.5, 512 rows 56.2 -> 33.9, 1000 rows 69.0 -> 49.0, 8192 rows 461 -> 310;
+// O 64 rows 55.2 -> 13.3, 512 rows 56.5 -> 29.3, 8192 rows 316 -> 225 (in the cache
+// 208: 1.32 PFLOP/s; a library product of 8192^3 on the same card reaches 1.28);
+// down 64 rows 160 -> 32.3, 512 rows 165 -> 77.4, 8192 rows 930 -> 622.
 // Against the general kernel, at the cheapest tile's shapes, tile / general: 256 x
 // 256 in the mean 0.92 (up to 1.05) at K = 384, 0.98 (1.11) at 256; 256 x 128 at once
 // 1.00 at 512, 0.97 at 640, in turn 1.05 at 256, 0.98 at 384; 128 x 192 1.20 at 384,

@@ -7,12 +7,13 @@ namespace {
 
 // Rows x weight rows of a tile, and the costs fitted to 57 shapes (N x K of
 // q|k|v 6144 x 4096, down 4096 x 12800, gate|up 25600 x 4096, 17 to 8192 rows,
-// us; the choice by them is within 2 % of the best of these at every one).
-// Measured against the 128 x 128 / 128 x 64 kernels of gemm.hip, us: q|k|v 64
-// rows 17.4 -> 8.7, 1000 rows 29.8 -> 25.7, 8192 rows 224 -> 164; down 64 rows
-// 41.5 -> 18.3, 512 rows 45.3 -> 34.3, 8192 rows 425 -> 320; gate|up 64 rows
-// 38.2 -> 24.0, 512 rows 80.6 -> 56.7, 8192 rows 867 -> 667 (2.58 PFLOP/s; a
-// library product of 8192^3 on the same card reaches 2.72).
+// us, the weights in the cache; the choice by them is within 2 % of the best of
+// these at every one). Measured against the 128 x 128 / 128 x 64 kernels of
+// gemm.hip, us, the operands rotated through 700 MB: q|k|v 64 rows 16.3 -> 12.2,
+// 1000 rows 39.1 -> 30.3, 8192 rows 231 -> 174; down 64 rows 39.6 -> 28.1, 512 rows
+// 49.7 -> 48.6, 1000 rows 94.5 -> 65.4, 8192 rows 436 -> 341; gate|up 64 rows 38.0 ->
+// 27.2, 512 rows 79.3 -> 62.0, 8192 rows 890 -> 708 (in the cache 667: 2.58 PFLOP/s;
+// a library product of 8192^3 on the same card reaches 2.72).
 // Against the general kernels, at the cheapest tile's shapes, tile / general:
 // 256 x 256 in the mean 0.93 (up to 1.08) at K = 1024, 0.96 (1.11) at 768; 256 x 128
 // at once 1.00-1.06 at 3584, 0.97-1.03 at 4096, in turn 1.00 at 2560, 0.96 at 3072;
@@ -32,7 +33,9 @@ constexpr TileConfig<true, 2, 2, 4, 2, false> k64x64{{6.45f, 3.33f, -0.57f}};
 constexpr TileConfig<true, 2, 1, 4, 2, false> k64x32{{4.95f, 1.45f, 1.16f}};
 constexpr TileCost kGeneral{29.20f, 3.99f, 0.02f};  // a round of 512 tiles
 // SwiGLU, whose general kernel has 128-row tiles of 64 columns only: 256 x 256 0.97
-// at 768, 1.03 at 512; the smaller ones faster from where they fit.
+// at 768, 1.03 at 512; the smaller ones faster from where they fit. Gate and up
+// rows in pairs need an even FN and whole loads of each: not 192, 96 or 32
+// columns; 128 x 64 was not measured for it.
 constexpr TileConfig<true, 8, 8, 2, 1, true> kGlu256x256{k256x256.cost, {768, 768, {44.14f, 7.63f, 3.00f}}};
 constexpr TileConfig<true, 8, 4, 3, 1, true> kGlu256x128{k256x128.cost, {4096, 3072, {25.38f, 4.54f, 2.40f}}};
 constexpr TileConfig<true, 4, 4, 4, 1, false> kGlu128x128{k128x128.cost, {0, 0, {15.84f, 1.68f, 2.69f}}};
