@@ -823,18 +823,25 @@ unsigned gemm_grid(long long tiles, int cap) {
 // CU (K = 12800 down, 8 rows, us: skinny 12.5, tile 14.6; bf16 O 7.4 / 9.1), but
 // re-reads all activations in each, which past that costs more than the
 // tile's staging, the sooner the more rows and K there are, and the later the
-// shorter the tile's K loop is (tile / skinny over 60 pairs of N and K from 4352
-// to 100352 columns, 1 to 16 rows):
-//   FP8 up to two per CU, M K >= 32768: 0.69-1.03; M K = 16384: 0.94-1.05, and
-//   1.12 where the weights come from memory (q|k|v 4 rows 9.6 / 10.7 us). More,
-//   M K >= 16384: 0.63-1.03; 4096: 1.00-1.28, 8192: 0.90-1.12. Past 32768 columns 4
-//   and 8 rows are 0.95-1.17, 12 and 16 0.79-1.00.
+// shorter the tile's K loop is. Where few of its workgroups are left for a last
+// round (spare: the CUs without one then), it is the slower one. With a K that is a
+// multiple of 8192, the rows of a tile whole 8 KB apart, the tile streams the weights
+// more slowly (FP8 25600 columns, 4 rows: tile / skinny 0.93 at K = 7168, 1.20 at 8192).
+// Tile / skinny from 4352 to 100352 columns, 1 to 16 rows, K of 768 to 12800, the
+// weights from memory as a layer's are in an engine:
+//   FP8 up to two per CU, M K >= 32768: 0.70-1.00 (M K = 16384: 1.12). Past that,
+//   M K >= 16384: 0.63-1.03, but 4 rows of K = 4096 1.09 and 1.11 without spare CUs.
+//   Past 32768 columns 12 and 16 rows 0.67-1.01, 4 and 8 0.95-1.17. K = 8192: 12 and 16
+//   rows 0.77-1.07, 8 rows 0.91-0.96 up to 6144 columns, 0.95-1.15 past them.
 //   bf16 up to two per CU, M K >= 16384: 0.65-1.01; M K = 8192: 0.95-1.13. Up to
-//   four, M K >= 768: 0.51-0.98. More: 4 rows and up 0.57-0.99, 2 rows 0.81-0.99 up
-//   to K = 4096 and 1.05-1.19 past it, 1 row 0.87-1.25.
-//   SwiGLU past two per CU, K >= 3584: 0.76-1.11; K = 2048: 1.00-1.28. Between one
-//   and a half and two 0.94-1.31. Up to one and a half, M K >= 256 for each
-//   workgroup past one per CU: 0.67-1.03.
+//   four, M K >= 768: 0.60-1.04. More: 0.60-1.00, 1 row 0.87-1.25. Below 4 rows, K of
+//   6144 and more: 1.09-1.14 up to three per CU, 0.92-0.98 up to four (K = 8192
+//   0.98-1.16), 0.99-1.19 past that.
+//   SwiGLU, K = 1024 and 2048: 0.98-1.28. Past two per CU up to four, by rows and
+//   spare CUs: 0.78-1.07 (32768 gate and up rows, no CU spare: 1 row 1.17, 8 rows 1.13,
+//   16 rows 1.04); past four 1.02-1.42, K = 8192 1.00-1.38. Between one and a half and
+//   two 0.94-1.31. Up to one and a half, M K >= 320 for each workgroup past one per
+//   CU: 0.81-1.04, K = 8192 three times as much: 0.82-1.02 (M K at 256: up to 1.15).
 // Where only tiles of 128 rows and more fit (K not a multiple of 512, bf16 of
 // 256), the skinny kernel is up to 3 times as fast.
 enum class GemmKind { kFp8, kBf16, kSwiglu };
@@ -843,16 +850,22 @@ bool skinny_rows(GemmKind kind, int M, int ncols, int K) {
   const int ntile = (ncols + 15) / 16;
   if (ntile <= kCUs || K % (kind == GemmKind::kBf16 ? 256 : 512) != 0) return true;
   const long long mk = static_cast<long long>(M) * K;
+  const bool pitch8k = K % 8192 == 0;
+  const int spare = kCUs - 1 - (ntile - 1) % kCUs;
   switch (kind) {
-    case GemmKind::kFp8: return mk < (ntile > 2 * kCUs ? 16384 : 32768) || M < (ntile > 8 * kCUs ? 12 : 4);
+    case GemmKind::kFp8:
+      if (ntile > 8 * kCUs) return M < 12;
+      if (pitch8k) return M < (ntile < 2 * kCUs ? 8 : 12);
+      return ntile > 2 * kCUs ? mk < 16384 || M < (K < 6144 && spare < 128 ? 8 : 4) : mk < 32768 || M < 4;
     case GemmKind::kSwiglu:
-      if (ntile > 2 * kCUs) return K < 3584;
-      return 2 * ntile > 3 * kCUs || K < 1024 || mk < 256LL * (ntile - kCUs);
+      if (K < 3584) return true;
+      if (ntile > 2 * kCUs) return pitch8k || ntile > 4 * kCUs || M + spare / 16 < 15;
+      return 2 * ntile > 3 * kCUs || mk < (pitch8k ? 768LL : 320LL) * (ntile - kCUs);
     default:
       if (K < 512) return true;
       if (ntile <= 2 * kCUs) return mk < 16384 || M < 4;
-      if (ntile <= 4 * kCUs) return mk < 768;
-      return M < 2 || (M < 4 && K > 4096);
+      if (M < 4 && K > 4096 && (ntile <= 3 * kCUs || ntile > 4 * kCUs || pitch8k)) return true;
+      return ntile <= 4 * kCUs ? mk < 768 : M < 2;
   }
 }
 

@@ -61,6 +61,20 @@ FASTER = [  # FP8 (None: SwiGLU), rows, columns, K, kernel
     (None, 300, 8192, 2560, "gemm_fp8_kernel"),     # 1.1
     (None, 300, 9600, 2560, "gemm_fp8_kernel"),     # 1.1
     (None, 8, 8192, 4096, "gemm_skinny_kernel"),    # 1.2
+    # weights from memory
+    (None, 8, 16384, 4096, "gemm_skinny_kernel"),   # 1.13
+    (None, 8, 12288, 4096, "gemm_skinny_kernel"),   # 1.08
+    (None, 1, 20480, 5120, "gemm_skinny_kernel"),   # 1.4
+    (None, 16, 12288, 8192, "gemm_skinny_kernel"),  # 1.2
+    (None, 8, 5120, 2048, "gemm_skinny_kernel"),    # 1.09
+    (None, 8, 6144, 8192, "gemm_skinny_kernel"),    # 1.08
+    (True, 4, 16384, 4096, "gemm_skinny_kernel"),   # 1.09
+    (True, 8, 16384, 8192, "gemm_skinny_kernel"),   # 1.15
+    (True, 4, 6144, 8192, "gemm_skinny_kernel"),    # 1.06
+    (False, 2, 9216, 6144, "gemm_skinny_kernel"),   # 1.09
+    (None, 16, 16384, 6144, "gemm_tile_kernel"), (None, 8, 12800, 4096, "gemm_tile_kernel"),
+    (None, 16, 6144, 4096, "gemm_tile_kernel"), (True, 4, 12800, 4096, "gemm_tile_kernel"),
+    (True, 12, 16384, 7168, "gemm_tile_kernel"), (False, 2, 12800, 6144, "gemm_tile_kernel"),
     (True, 2561, 6144, 4096, "gemm_fp8_kernel"),    # 1.3
     (None, 832, 12800, 4096, "gemm_fp8_kernel"),    # 1.08
     (True, 512, 4096, 12800, "gemm_tile_kernel"), (True, 8192, 6144, 4096, "gemm_tile_kernel"),
