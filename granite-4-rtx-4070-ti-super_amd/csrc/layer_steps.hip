@@ -146,9 +146,9 @@ int qkv_gemm(const Granite4DecodeModel* m, const Granite4DecodeLayer& y,
   // Rows of a weight block into buffers of their own: one launch, the same sums
   // as a call per matrix where those take the skinny kernel too. Past 4096
   // columns they may not: a model with that many q columns (more than 32
-  // heads) takes a tile for q, and the one launch for k and v (H 4096, 40
-  // heads, per layer at short contexts, us: 4 rows 63 -> 67 FP8, 69 bf16; 16
-  // rows 74 -> 77, 77 -> 82; 32 heads unchanged).
+  // heads) takes a tile for q from some rows on, and the one launch for k and v
+  // (H 4096, 40 heads, per layer at short contexts, us: 16 rows 74 -> 77 FP8, 77
+  // -> 82 bf16; FP8 below 8 rows and 32 heads unchanged).
   const bool contiguous_w = y.wk == y.wq + static_cast<size_t>(nq) * H &&
                             y.wv == y.wk + static_cast<size_t>(nk) * H;
   const bool split = contiguous_w && rows <= kSkinnyRows && g4::gemm_rows_skinny(fp8, rows, nk, H);
