@@ -33,6 +33,7 @@ struct GemmArgs {
   int mt, nt;       // tile counts along M and N
   bool vec_out;     // 16-byte output rows (pitch and width multiples of 8)
   bool xcd_order;   // tiles renumbered per XCD (xcd_tile0)
+  bool n_major;     // tile kernel: consecutive tiles are one row of them, not one column
   // Skinny kBf16 only (gemm_rows_split): when seg_out[0] is set, column n of
   // segment s (ep.seg1 / ep.seg2 bounds) goes to seg_out[s][m * seg_ld[s] +
   // n - start of s] instead of ep.out_bf16.
@@ -67,6 +68,25 @@ inline bool gemm_xcd_order(int mt, unsigned g) {
   const long long xbm = mt < per ? mt : per, xbn = (per + mt - 1) / mt;
   const long long pbm = mt <= 8 ? 1 : mt / 8, pbn = mt <= 8 ? per : (g + mt - 1) / mt;
   return xbm + xbn < pbm + pbn;
+}
+
+// Whether the tile kernel, where gemm_xcd_order keeps the plain order, numbers
+// its tiles along N (consecutive tiles share their A rows) and gives each XCD
+// consecutive ones. In the plain order an XCD runs every 8th tile of a column of
+// mt: mt / 8 M tiles only where 8 divides mt, all of them where mt is odd, as it
+// often is with 256-row tiles, and every XCD then reads all of A. Along N it covers
+// g / 8 tiles of a row and the next ones. Taken where that block is at most 4/5 of
+// the plain order's. FP8, us, the operands from memory: N x K of 1024 x 4096, 6337
+// rows 40 -> 29 (general kernel 31), 7936 rows 47 -> 32 (35); 3072 x 4096, 7936 rows
+// 129 -> 91 (107); 6144 x 4096, 6200 rows 187 -> 153; bf16 4096 x 12800, 4900 rows 650 ->
+// 501. A block nearly as large is no gain: 25600 x 4096 0.99-1.12.
+inline bool gemm_n_major(int mt, int nt, unsigned g) {
+  if (g < 16) return false;
+  const long long per = g / 8, cols = (static_cast<long long>(g) + mt - 1) / mt;
+  const long long every = mt % 8 == 0 ? mt / 8 : mt % 4 == 0 ? mt / 4 : mt % 2 == 0 ? mt / 2 : mt;
+  const long long plain = (every < per ? every : per) + (cols < per ? cols : per);
+  const long long along = (per + nt - 1) / nt + (nt < per ? nt : per);
+  return 5 * along <= 4 * plain;
 }
 
 __device__ __forceinline__ float epi_scale(const Granite4GemmEpilogue& ep, int n) {

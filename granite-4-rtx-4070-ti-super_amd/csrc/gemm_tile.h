@@ -142,6 +142,12 @@ __device__ __forceinline__ int tile_swz128(int r) { return (r >> 1) & 7; }
 __device__ __forceinline__ int tile_swz64(int r) { return (r >> 2) & 3; }
 #endif
 
+// (M tile, N tile) of a tile number.
+__device__ __forceinline__ int2 tile_at(const GemmArgs& a, int tile) {
+  const int d = a.n_major ? a.nt : a.mt, q = tile / d, r = tile - q * d;
+  return a.n_major ? make_int2(q, r) : make_int2(r, q);
+}
+
 template <bool F8, int EPI, int FM, int FN, int S, int KS, bool QUAD>
 __global__ __launch_bounds__(256 * KS) __attribute__((amdgpu_waves_per_eu(KS, KS))) void gemm_tile_kernel(GemmArgs a) {
 #ifdef __HIP_DEVICE_COMPILE__  // the host pass needs the launch stub only
@@ -196,7 +202,8 @@ __global__ __launch_bounds__(256 * KS) __attribute__((amdgpu_waves_per_eu(KS, KS
   const auto col_of = [&](int r) { return kGlu ? r / (16 * FN) * (8 * FN) + r % (8 * FN) : r; };
   static_assert(!kGlu || (8 * FN) % kWRows == 0 || kWRows % (16 * FN) == 0, "a load's columns follow its rows");
   const auto source = [&](Source& s, int tile) __attribute__((always_inline)) {
-    const int m0 = (tile % a.mt) * T::kBM, n0 = (tile / a.mt) * kTileCols;
+    const int2 at = tile_at(a, tile);
+    const int m0 = at.x * T::kBM, n0 = at.y * kTileCols;
     s.abase = a.A + static_cast<size_t>(m0) * apitch + static_cast<size_t>(kg * steps) * 128;
     s.wbase = a.W + static_cast<size_t>(n0) * a.K + static_cast<size_t>(kg * steps) * T::kKb;
     s.ao = static_cast<uint32_t>(ar0 * apitch) + ac;
@@ -423,7 +430,8 @@ __global__ __launch_bounds__(256 * KS) __attribute__((amdgpu_waves_per_eu(KS, KS
 #pragma unroll
     for (int q = 0; q < FM * FN; ++q) asm volatile("" : "+a"(acc[q / FN][q % FN]));
 
-    const int m0 = (tile % a.mt) * T::kBM, n0 = (tile / a.mt) * kTileCols;
+    const int2 at = tile_at(a, tile);
+    const int m0 = at.x * T::kBM, n0 = at.y * kTileCols;
     constexpr int kSlot = 4 * FM * FN * 64;  // between the K groups' hand-overs
     if constexpr (KS > 1) {
       // The K groups' partial sums meet, in group order: group b % KS finishes
@@ -658,6 +666,8 @@ struct TileConfig {
     a.nt = ((kGlu ? a.I : a.N) + cols(kGlu) - 1) / cols(kGlu);
     const unsigned grid = static_cast<unsigned>(t < kCUs ? t : kCUs);
     a.xcd_order = gemm_xcd_order(a.mt, grid);
+    a.n_major = !a.xcd_order && gemm_n_major(a.mt, a.nt, grid);
+    a.xcd_order = a.xcd_order || a.n_major;
     hipLaunchKernelGGL((gemm_tile_kernel<F8, EPI, FM, FN, S, KS, QUAD>), grid, 256 * KS, 0, stream(), a);
     return grid;
   }

@@ -14,14 +14,15 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 ADDR = 0x10000000  # any 16-byte aligned address
 
 
-def launched(steps):
+def launched(steps, want="launches"):
     """Per step, the launches [(kernel, grid, threads)]. A step is a function
-    of `Steps` and its arguments: ("gemm", True, 512, 4096, 4096)."""
+    of `Steps` and its arguments: ("gemm", True, 512, 4096, 4096). want="orders":
+    [(M tiles, N tiles, numbered per XCD, numbered along N)] of tile GEMMs."""
     with tempfile.TemporaryDirectory() as d:
         stub = os.path.join(d, "libhipstub.so")
         subprocess.run(["gcc", "-O1", "-shared", "-fPIC", "-o", stub, os.path.join(HERE, "hip_stub.c")],
                        check=True)
-        r = subprocess.run([sys.executable, os.path.abspath(__file__), stub], input=json.dumps(steps),
+        r = subprocess.run([sys.executable, os.path.abspath(__file__), stub, want], input=json.dumps(steps),
                            capture_output=True, text=True, timeout=300)
     assert r.returncode == 0, r.stderr[-2000:]
     return json.loads(r.stdout)
@@ -45,6 +46,18 @@ class Steps:
         sys.path.insert(0, HERE)
         from pkg import layerops
         self.L = layerops()
+
+    def order(self, address):
+        """The tile counts and orders in a tile GEMM's argument (GemmArgs)."""
+        c, p, i = ctypes, ctypes.c_void_p, ctypes.c_int
+
+        class Args(c.Structure):
+            _fields_ = [("A", p), ("lda", i), ("a_scale", p), ("W", p), ("M", i), ("N", i), ("K", i), ("I", i),
+                        ("ep", self.L.GemmEpilogue), ("partials", p), ("mt", i), ("nt", i), ("vec_out", c.c_bool),
+                        ("xcd_order", c.c_bool), ("n_major", c.c_bool)]
+
+        a = Args.from_address(address)
+        return a.mt, a.nt, a.xcd_order, a.n_major
 
     def _ep(self, n):
         return self.L.GemmEpilogue(1.0, 1.0, 1.0, n, n, ADDR, ADDR, ADDR, 1.0, n)
@@ -86,6 +99,7 @@ class Steps:
 def _child():
     stub = ctypes.CDLL(sys.argv[1], mode=ctypes.RTLD_GLOBAL)
     stub.stub_name.restype = ctypes.c_char_p
+    stub.stub_arg.restype = ctypes.c_void_p
     s, out = Steps(stub), []
     for name, *args in json.load(sys.stdin):
         stub.stub_reset()
@@ -94,7 +108,8 @@ def _child():
         for i in range(stub.stub_launches()):
             g = (ctypes.c_uint * 4)()
             stub.stub_grid(i, g)
-            got.append((stub.stub_name(i).decode(), list(g[:3]), g[3]))
+            got.append(s.order(stub.stub_arg(i)) if sys.argv[2] == "orders" else
+                       (stub.stub_name(i).decode(), list(g[:3]), g[3]))
         assert stub.stub_pool_allocs() == stub.stub_pool_frees()
         out.append(got)
     print(json.dumps(out))

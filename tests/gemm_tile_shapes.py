@@ -25,6 +25,9 @@ FP8 = [
     (33, 40, 1536, (2, 1), 1),
     (17, 8, 1024, (2, 1), 1),
     (16, 6152, 2048, (2, 1), 1),      # 16 rows, more skinny workgroups than CUs
+    (2053, 520, 1024, (2, 3), 1),     # tiles numbered along N from here on
+    (2820, 1032, 1536, (4, 4), 1),
+    (6700, 4104, 1024, (8, 8), 2),    # 459 tiles
 ]
 BF16 = [
     (257, 16392, 512, (8, 8), 1),
@@ -46,6 +49,9 @@ BF16 = [
     (33, 42, 1024, (1, 2), 1),
     (17, 40, 2048, (1, 1), 1),        # four K groups
     (9, 8200, 512, (2, 2), 1),        # 9 rows, more skinny workgroups than CUs
+    (2053, 520, 512, (2, 4), 1),      # tiles numbered along N from here on
+    (2307, 2054, 512, (4, 6), 1),
+    (6700, 3078, 512, (8, 4), 3),     # 675 tiles
 ]
 SWIGLU = [
     (17, 16392, 768, (8, 8), 1),
@@ -60,6 +66,8 @@ SWIGLU = [
     (17, 40, 1024, (2, 2), 1),
     (300, 520, 1536, (2, 2), 1),
     (16, 8264, 3584, (2, 4), 1),      # 16 rows, more skinny workgroups than CUs
+    (2820, 520, 512, (4, 4), 1),      # tiles numbered along N from here on
+    (6700, 2056, 1024, (8, 8), 2),    # 459 tiles
 ]
 # K too short for a tile, or fewer rows than it takes: the general and the skinny kernels.
 FP8_OTHER = [(17, 40, 256), (17, 136, 512), (2049, 2600, 256), (700, 8200, 512), (129, 8200, 1024),

@@ -5,12 +5,13 @@
 #include <stddef.h>
 #include <stdint.h>
 #include <stdlib.h>
+#include <string.h>
 
 typedef struct {
   unsigned x, y, z;
 } Dim3;
 
-enum { kMax = 4096, kOk = 0, kErr = 2 /* hipErrorOutOfMemory */ };
+enum { kMax = 4096, kArgBytes = 128, kOk = 0, kErr = 2 /* hipErrorOutOfMemory */ };
 
 static struct {
   const void* host;
@@ -21,6 +22,7 @@ static int kernel_count;
 static struct {
   const char* name;
   Dim3 grid, block;
+  char arg[kArgBytes]; /* of the tile GEMM: the start of its argument */
 } launches[kMax];
 static int launch_count, pool_fails, capturing, pool_allocs, pool_frees;
 
@@ -43,6 +45,8 @@ void stub_grid(int i, unsigned* out) {
   out[2] = launches[i].grid.z;
   out[3] = launches[i].block.x;
 }
+
+const char* stub_arg(int i) { return launches[i].arg; }
 
 void** __hipRegisterFatBinary(const void* data) {
   static void* handle;
@@ -76,12 +80,13 @@ int __hipPopCallConfiguration(Dim3* grid, Dim3* block, size_t* shared, void** st
   return kOk;
 }
 int hipLaunchKernel(const void* f, Dim3 grid, Dim3 block, void** args, size_t shared, void* stream) {
-  (void)args, (void)shared, (void)stream;
+  (void)shared, (void)stream;
   const char* name = "?";
   for (int i = 0; i < kernel_count; ++i)
     if (kernels[i].host == f) name = kernels[i].name;
   if (launch_count < kMax) {
     launches[launch_count].name = name;
+    if (strstr(name, "gemm_tile_kernel") != NULL) memcpy(launches[launch_count].arg, args[0], kArgBytes);
     launches[launch_count].grid = grid;
     launches[launch_count++].block = block;
   }

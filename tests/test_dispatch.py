@@ -139,11 +139,27 @@ def test_gemm_tile_shapes_run_the_named_tiles():
         assert (name, tuple(args[2:4])) == ("gemm_tile_kernel", fragments), (fp8, m, n, k)
         count = shapes.tiles(m, n, fragments, fp8 is None)
         assert grid == min(count, 256) and -(-count // grid) == turns, (fp8, m, n, k, count)
+    along_n = [t for t, o in zip(todo, launched([step(*t[:4]) for t in todo], "orders")) if o[0][3]]
+    assert along_n == [(True, *s) for s in shapes.FP8[-3:]] + [(False, *s) for s in shapes.BF16[-3:]] + [
+        (None, *s) for s in shapes.SWIGLU[-2:]]
     other = [step(t[0], t[1], t[2], t[3] + (32 if t[0] is False else 128)) for t in todo]
     other += [step(f, *s) for f, l in ((True, shapes.FP8_OTHER), (False, shapes.BF16_OTHER),
                                        (None, shapes.SWIGLU_OTHER)) for s in l]
     for s, got in zip(other, launched(other)):
         assert kernel(got[0][0])[0] != "gemm_tile_kernel", s
+
+
+# Where an XCD would run every 8th tile of a column with an odd number of them,
+# and so read all of A, tiles are numbered along N (us plain / along N).
+@pytest.mark.parametrize("fp8,m,n,k,order", [
+    (True, 6337, 1024, 4096, (25, 8, True, True)),      # 40 / 29
+    (True, 7936, 3072, 4096, (31, 24, True, True)),     # 129 / 91
+    (False, 7936, 4096, 12800, (31, 16, True, True)),   # 602 / 578
+    (True, 8192, 4096, 12800, (32, 16, False, False)),  # an eighth of the M tiles per XCD
+    (True, 6337, 25600, 4096, (25, 100, False, False)),  # along N as much of W as of A before
+    (True, 512, 4096, 12800, (4, 64, True, False))])
+def test_gemm_tile_order(fp8, m, n, k, order):
+    assert [tuple(o) for o in launched([("gemm", fp8, m, n, k)], "orders")[0]] == [order]
 
 
 # The bf16 general kernel's two residual forms: loaded at a tile's start, or
